@@ -4,13 +4,6 @@
 
 using namespace mitos;
 
-namespace mitos {
-
-template struct Pipe<float>;
-template struct Pipe<double>;
-
-}  // namespace mitos
-
 // ---- C API ------------------------------------------------------------------------------
 struct mitos_ic_context {
     int N;
