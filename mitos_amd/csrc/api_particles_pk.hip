@@ -11,6 +11,7 @@
 
 #include "../../include/mitos_hip.h"
 #include "api_util.h"
+#include "cic_sort.h"
 #include "particles.h"
 #include "powerspec.h"
 
@@ -271,8 +272,17 @@ extern "C" int mitos_cic_overdensity(int N, double boxlen, long long npart, cons
     if (!grid) return set_last_error(MITOS_ERR_ALLOC);
     hipStream_t s = api_stream();
     MITOS_HIP_CHECK(hipMemsetAsync(grid, 0, sizeof(unsigned long long) * ncell, s));
-    hipLaunchKernelGGL(k_cic<double>, dim3(nblk(npart)), dim3(256), 0, s, X, Y, Z, npart, N, boxlen,
-                       grid);
+    // sorted by tile when that pays and its buffers can be had, else one atomic
+    // per corner of every particle: the same integers
+    const size_t sort_bytes = cic_sort_bytes(N, npart);
+    void* sort_ws = cic_sort_pays(N, npart) ? workspace(8, sort_bytes) : nullptr;
+    if (!sort_ws) (void)hipGetLastError();  // no room for the sort: the atomics need none
+    if (sort_ws)
+        MITOS_TRY(set_last_error(
+            cic_sorted<double>(X, Y, Z, npart, N, boxlen, grid, sort_ws, sort_bytes, s)));
+    else
+        hipLaunchKernelGGL(k_cic<double>, dim3(nblk(npart)), dim3(256), 0, s, X, Y, Z, npart, N,
+                           boxlen, grid);
     MITOS_TRY(set_last_error(launch_status()));
     const double norm = ldexp(1.0, -MITOS_CIC_SHIFT) * ((double)ncell / (double)npart);
     hipLaunchKernelGGL((k_cic_to_delta<double>), dim3(nblk(ncell)), dim3(256), 0, s, grid, box,

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/mitos_hip.h"
+#include "cic_sort.h"
 #include "pipeline_kernels.h"
 #include "powerspec.h"
 

@@ -473,6 +473,11 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
                                                             nullptr, s)));
                     return launch_status();
                 }
+                // another lattice than the grid's: sorted by tile, in the A grids
+                // (free once the displacement grids are made)
+                if (cic_sort_pays(NN, nl))
+                    return cic_sorted<M>(X, Y, Z, nl, NN, L, cic(), A,
+                                         sizeof(cx<T>) * (size_t)csize * 3, s);
                 hipLaunchKernelGGL(k_cic<M>, dim3(nblk(nl)), dim3(256), 0, s, X, Y, Z, nl, NN, L,
                                    cic());
                 return launch_status();
