@@ -61,115 +61,261 @@ __global__ void k_fill(T* p, long n, T v) {
     if (i < n) p[i] = v;
 }
 
-__device__ __forceinline__ void wrap3(int c, int N, float invN, int o[3]) {
-    const int b = wrapf(c, N, invN);
-    o[0] = b == 0 ? N - 1 : b - 1;
-    o[1] = b;
-    o[2] = b == N - 1 ? 0 : b + 1;
-}
-
-// Per lattice particle: the moves of k_move_deposit_s recomputed in T, the
-// CIC adjoint at the final position, then the adjoint of the three moves.
-// sx, sy, sz: the stencilled displacement grids (halo rows of rs); grho, A*:
-// dense N^3 grids.
-// The y and z move adjoints scatter to neighbouring x (and y) lattice rows.
-// The scatter is made order-independent (bit-reproducible gradients) in
-// fixed point: pass 0 finds max|gy| and max|gz| (an integer maximum of the
-// doubles' bit patterns), pass 1 adds -g w in units of max * 2^-48 to 64-bit
-// integer grids (at most 2^15 maximal contributions per cell before overflow),
-// and k_adj_fixed_to_real converts them.
+// bits of the fixed-point sums of the scatter adjoint below the largest gradient
 constexpr int kAdjFixedBits = 48;
 
-template <typename T, int PASS>
+// the larger magnitude; a NaN stays
+template <typename T>
+__device__ __forceinline__ T adj_max(T m, T a) {
+    return (a > m || a != a) ? a : m;
+}
+
+// Adjoint of the particles, in two passes over 8 x 8 x 16 lattice tiles.
+// sx, sy, sz: the stencilled displacement grids (rows of rs); grho, Ax, gy, gz:
+// dense N^3 grids.
+//
+// k_adj_gradients, per particle: the three moves recomputed in T with the
+// position derivatives of their taps, the CIC adjoint at the final position,
+// and from them dL/dx, dL/dy, dL/dz of the moves: Ax = -dL/dx (the x move reads
+// its own site alone), gy and gz to memory.  Each work-group leaves the largest
+// |gy| and |gz| in part: two atomic maxima per particle queued at one line, 6.0
+// ms at 256^3 in FP32 against 0.54 ms now, bound by the 21 tap loads.
+template <typename T>
 __global__ void __launch_bounds__(256)
-    k_adj_particles(const T* __restrict__ sx, const T* __restrict__ sy,
-                    const T* __restrict__ sz, unsigned rs, const T* __restrict__ grho, T* Ax,
-                    unsigned long long* AyI, unsigned long long* AzI,
-                    unsigned long long* gmax, int N, double boxlen, float spacing) {
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long n = (long long)N * N * N;
-    if (p >= n) return;
-    const int qz = (int)(p % N);
-    const int qy = (int)((p / N) % N);
-    const int qx = (int)(p / ((long long)N * N));
+    k_adj_gradients(const T* __restrict__ sx, const T* __restrict__ sy, const T* __restrict__ sz,
+                    unsigned rs, const T* __restrict__ grho, T* __restrict__ Ax,
+                    T* __restrict__ gyo, T* __restrict__ gzo, double* __restrict__ part, int N,
+                    double boxlen, float spacing) {
+    __shared__ double red[2][4];
+    int x0, y0, z0;
+    adj_tile(xcd_block(blockIdx.x, gridDim.x), N, x0, y0, z0);
+    const int qz = z0 + (int)(threadIdx.x & 15), qy = y0 + (int)((threadIdx.x >> 4) & 7);
     const T Lb = (T)boxlen, sN = (T)(N / boxlen);
-    T x1, y1, z1;
-    moves_s(sx, sy, sz, rs, N, sN, spacing, qx, qy, qz, x1, y1, z1);
-    // CIC (analyse/src/mitos_read.c:285-320): d rho(corner) / d position
-    int iX, iY, iZ;
-    T dx, dy, dz;
-    cic_cell_t(wrap_pos(x1, Lb), sN, N, iX, dx);
-    cic_cell_t(wrap_pos(y1, Lb), sN, N, iY, dy);
-    cic_cell_t(wrap_pos(z1, Lb), sN, N, iZ, dz);
-    const long x0 = wrapi(iX, N), xp = wrap1((int)x0 + 1, N);
-    const long y0 = wrapi(iY, N), yp = wrap1((int)y0 + 1, N);
-    const long z0 = wrapi(iZ, N), zp = wrap1((int)z0 + 1, N);
-    auto g = [&](long a, long b, long c) { return grho[(a * N + b) * N + c]; };
-    const T g000 = g(x0, y0, z0), g100 = g(xp, y0, z0), g010 = g(x0, yp, z0),
-            g001 = g(x0, y0, zp), g110 = g(xp, yp, z0), g101 = g(xp, y0, zp),
-            g011 = g(x0, yp, zp), g111 = g(xp, yp, zp);
-    const T tx = 1 - dx, ty = 1 - dy, tz = 1 - dz;
-    const T gX = sN * (ty * tz * (g100 - g000) + dy * tz * (g110 - g010) +
-                       ty * dz * (g101 - g001) + dy * dz * (g111 - g011));
-    const T gY = sN * (tx * tz * (g010 - g000) + dx * tz * (g110 - g100) +
-                       tx * dz * (g011 - g001) + dx * dz * (g111 - g101));
-    const T gZ = sN * (tx * ty * (g001 - g000) + dx * ty * (g101 - g100) +
-                       tx * dy * (g011 - g010) + dx * dy * (g111 - g110));
-    // moves: x1 = x0 - Sx(q), y1 = y0 - Fy(x1), z1 = z0 - Fz(x1, y1)
     const float invN = 1.0f / N;
-    int cx, cy;
-    T wx[3], dwx[3], wy[3], dwy[3];
-    tsc_axis_near_d(x1 * sN, cx, wx, dwx);
-    tsc_axis_near_d(y1 * sN, cy, wy, dwy);
-    int ix[3], iy[3];
-    wrap3(cx, N, invN, ix);
-    wrap3(cy, N, invN, iy);
-    const unsigned zo = MITOS_PSI_SO + qz;
-    T Fy_x = 0, Fz_x = 0, Fz_y = 0;
+    const unsigned plane = (unsigned)N * rs, zo = MITOS_PSI_SO + qz;
+    T my = 0, mz = 0;
+    if (qz < N) {
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-        const unsigned ra = (unsigned)ix[a] * N;
-        Fy_x += dwx[a] * sy[(ra + qy) * rs + zo];
+        for (int j = 0; j < 4; j++) {
+            const int qx = x0 + (int)(threadIdx.x >> 7) + 2 * j;
+            const unsigned yz = (unsigned)qy * rs + zo;
+            // x1 = x0 - Sx(q), y1 = y0 - Fy(x1), z1 = z0 - Fz(x1, y1), with
+            // dFy/dx, dFz/dx and dFz/dy from the same taps
+            const T x1 = (T)(qx * spacing) - sx[(unsigned)qx * plane + yz];
+            int cx, cy;
+            T wx[3], dwx[3], wy[3], dwy[3];
+            unsigned ox[3], oy[3];
+            tsc_axis_near_d(x1 * sN, cx, wx, dwx);
+            tap_rows(wrapf(cx, N, invN), N, plane, ox);
+            T y1 = (T)(qy * spacing), z1 = (T)(qz * spacing), fy = 0, Fy_x = 0;
 #pragma unroll
-        for (int b = 0; b < 3; b++) {
-            const T v = sz[(ra + iy[b]) * rs + zo];
-            Fz_x += dwx[a] * wy[b] * v;
-            Fz_y += wx[a] * dwy[b] * v;
+            for (int a = 0; a < 3; a++) {
+                const T v = sy[ox[a] + yz];
+                fy += wx[a] * v;
+                Fy_x += dwx[a] * v;
+            }
+            y1 -= fy;
+            tsc_axis_near_d(y1 * sN, cy, wy, dwy);
+            tap_rows(wrapf(cy, N, invN), N, rs, oy);
+            T fz = 0, Fz_x = 0, Fz_y = 0;
+#pragma unroll
+            for (int a = 0; a < 3; a++)
+#pragma unroll
+                for (int b = 0; b < 3; b++) {
+                    const T v = sz[ox[a] + oy[b] + zo];
+                    fz += wx[a] * wy[b] * v;
+                    Fz_x += dwx[a] * wy[b] * v;
+                    Fz_y += wx[a] * dwy[b] * v;
+                }
+            z1 -= fz;
+            // CIC (analyse/src/mitos_read.c:285-320): d rho(corner) / d position
+            int iX, iY, iZ;
+            T dx, dy, dz;
+            cic_cell_t(wrap_pos(x1, Lb), sN, N, iX, dx);
+            cic_cell_t(wrap_pos(y1, Lb), sN, N, iY, dy);
+            cic_cell_t(wrap_pos(z1, Lb), sN, N, iZ, dz);
+            auto wrapped = [&](int i) { return (unsigned)i < (unsigned)N ? i : wrapi(i, N); };
+            const int cx0 = wrapped(iX), cxp = wrap1(cx0 + 1, N);
+            const int cy0 = wrapped(iY), cyp = wrap1(cy0 + 1, N);
+            const int cz0 = wrapped(iZ), czp = wrap1(cz0 + 1, N);
+            auto g = [&](int a, int b, int c) { return grho[((size_t)a * N + b) * N + c]; };
+            const T g000 = g(cx0, cy0, cz0), g100 = g(cxp, cy0, cz0), g010 = g(cx0, cyp, cz0),
+                    g001 = g(cx0, cy0, czp), g110 = g(cxp, cyp, cz0), g101 = g(cxp, cy0, czp),
+                    g011 = g(cx0, cyp, czp), g111 = g(cxp, cyp, czp);
+            const T tx = 1 - dx, ty = 1 - dy, tz = 1 - dz;
+            const T gX = sN * (ty * tz * (g100 - g000) + dy * tz * (g110 - g010) +
+                               ty * dz * (g101 - g001) + dy * dz * (g111 - g011));
+            const T gY = sN * (tx * tz * (g010 - g000) + dx * tz * (g110 - g100) +
+                               tx * dz * (g011 - g001) + dx * dz * (g111 - g101));
+            const T gZ = sN * (tx * ty * (g001 - g000) + dx * ty * (g101 - g100) +
+                               tx * dy * (g011 - g010) + dx * dy * (g111 - g110));
+            const T gz = gZ;
+            const T gy = gY - gz * Fz_y * sN;
+            const T gx = gX - gz * Fz_x * sN - gy * Fy_x * sN;
+            const size_t p = ((size_t)qx * N + qy) * N + qz;
+            Ax[p] = -gx;
+            gyo[p] = gy;
+            gzo[p] = gz;
+            my = adj_max(my, (T)fabs(gy));
+            mz = adj_max(mz, (T)fabs(gz));
         }
     }
-    const T gz = gZ;
-    const T gy = gY - gz * Fz_y * sN;
-    const T gx = gX - gz * Fz_x * sN - gy * Fy_x * sN;
-    if constexpr (PASS == 0) {
-        // positive doubles order as their bit patterns
-        atomicMax(gmax, (unsigned long long)__double_as_longlong(fabs((double)gy)));
-        atomicMax(gmax + 1, (unsigned long long)__double_as_longlong(fabs((double)gz)));
-        return;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        my = adj_max(my, __shfl_xor(my, o, 64));
+        mz = adj_max(mz, __shfl_xor(mz, o, 64));
     }
-    const double my = __longlong_as_double((long long)gmax[0]);
-    const double mz = __longlong_as_double((long long)gmax[1]);
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = (double)my;
+        red[1][threadIdx.x >> 6] = (double)mz;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double m = red[threadIdx.x][0];
+        for (int w = 1; w < 4; w++) m = adj_max(m, red[threadIdx.x][w]);
+        part[2 * blockIdx.x + threadIdx.x] = m;
+    }
+}
+
+// gmax[0], gmax[1] = largest of the n pairs of part; one work-group
+static __global__ void __launch_bounds__(1024)
+    k_adj_max(const double* __restrict__ part, unsigned n, double* gmax) {
+    __shared__ double red[2][16];
+    double m[2] = {0, 0};
+    for (unsigned i = threadIdx.x; i < n; i += 1024)
+        for (int q = 0; q < 2; q++) m[q] = adj_max(m[q], part[2 * i + q]);
+    for (int q = 0; q < 2; q++) {
+        for (int o = 32; o >= 1; o >>= 1) m[q] = adj_max(m[q], __shfl_xor(m[q], o, 64));
+        if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = m[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double v = red[threadIdx.x][0];
+        for (int w = 1; w < 16; w++) v = adj_max(v, red[threadIdx.x][w]);
+        gmax[threadIdx.x] = v;
+    }
+}
+
+// k_adj_scatter: the y and z move adjoints go to the x rows, and x and y rows,
+// that the moves read: -g w in units of max|g| 2^-48 to 64-bit integers (at most
+// 2^15 maximal contributions per cell before overflow), so the sums do not
+// depend on their order and gradients are bit-reproducible;
+// k_adj_fixed_to_real converts them.  Twelve global atomics per particle were
+// bound by the memory-side atomic units (5.8 ms at 256^3 in FP32); here a tile
+// sums in LDS windows placed at its mean displacement, four cells of margin on
+// each side, and adds whole rows of 16 z to the grids (0.56 ms).  A particle past
+// the margin takes the global atomics.
+template <typename T>
+__global__ void __launch_bounds__(512)
+    k_adj_scatter(const T* __restrict__ sx, const T* __restrict__ sy, unsigned rs,
+                  const T* __restrict__ gyi, const T* __restrict__ gzi, unsigned long long* AyI,
+                  unsigned long long* AzI, const double* __restrict__ gmax, int N, double boxlen,
+                  float spacing) {
+    constexpr int MARGIN = 4, WX = kAdjTX + 2 * (MARGIN + 1), TZ = kAdjTZ;
+    __shared__ unsigned long long winz[WX * WX * TZ];
+    __shared__ unsigned long long winy[WX * kAdjTY * TZ];
+    __shared__ int red[2][8];
+    int x0, y0, z0;
+    adj_tile(xcd_block(blockIdx.x, gridDim.x), N, x0, y0, z0);
+    const int lz = threadIdx.x & 15, ly = (threadIdx.x >> 4) & 7;
+    const int qz = z0 + lz, qy = y0 + ly;
+    const bool ok = qz < N;
+    for (int i = threadIdx.x; i < WX * WX * TZ; i += 512) winz[i] = 0;
+    for (int i = threadIdx.x; i < WX * kAdjTY * TZ; i += 512) winy[i] = 0;
+    const T sN = (T)(N / boxlen);
+    const float invN = 1.0f / N;
+    const unsigned plane = (unsigned)N * rs, yz = (unsigned)qy * rs + MITOS_PSI_SO + qz;
+    int cx[2], cy[2], sumx = 0, sumy = 0;
+    T wx[2][3], wy[2][3], gy[2], gz[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int qx = x0 + (int)(threadIdx.x >> 7) + 4 * j;
+        cx[j] = qx;
+        cy[j] = qy;
+        gy[j] = gz[j] = 0;
+        if (!ok) continue;
+        const size_t p = ((size_t)qx * N + qy) * N + qz;
+        gy[j] = gyi[p];
+        gz[j] = gzi[p];
+        const T x1 = (T)(qx * spacing) - sx[(unsigned)qx * plane + yz];
+        tsc_axis_near(x1 * sN, cx[j], wx[j]);
+        unsigned ox[3];
+        tap_rows(wrapf(cx[j], N, invN), N, plane, ox);
+        T fy = 0;
+#pragma unroll
+        for (int a = 0; a < 3; a++) fy += wx[j][a] * sy[ox[a] + yz];
+        const T y1 = (T)(qy * spacing) - fy;
+        tsc_axis_near(y1 * sN, cy[j], wy[j]);
+        sumx += cx[j] - qx;
+        sumy += cy[j] - qy;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        sumx += __shfl_xor(sumx, o, 64);
+        sumy += __shfl_xor(sumy, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = sumx;
+        red[1][threadIdx.x >> 6] = sumy;
+    }
+    __syncthreads();
+    sumx = sumy = 0;
+    for (int w = 0; w < 8; w++) {
+        sumx += red[0][w];
+        sumy += red[1][w];
+    }
+    const int wx0 = x0 + (int)rintf((float)sumx / 1024) - MARGIN - 1;
+    const int wy0 = y0 + (int)rintf((float)sumy / 1024) - MARGIN - 1;
+    const double my = gmax[0], mz = gmax[1];
     const double sy_ = my > 0 ? ldexp(1.0, kAdjFixedBits) / my : 0.0;
     const double sz_ = mz > 0 ? ldexp(1.0, kAdjFixedBits) / mz : 0.0;
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-        const long ra = (long)ix[a] * N;
-        atomicAdd(AyI + (ra + qy) * N + qz,
-                  (unsigned long long)llrint((double)(-gy * wx[a]) * sy_));
+    for (int j = 0; j < 2; j++) {
+        if (!ok) continue;
+        const int ax = cx[j] - 1 - wx0, ay = cy[j] - 1 - wy0;
+        const bool inx = ax >= 0 && ax + 2 < WX, in = inx && ay >= 0 && ay + 2 < WX;
 #pragma unroll
-        for (int b = 0; b < 3; b++)
-            atomicAdd(AzI + (ra + iy[b]) * N + qz,
-                      (unsigned long long)llrint((double)(-gz * wx[a] * wy[b]) * sz_));
+        for (int a = 0; a < 3; a++) {
+            const unsigned long long vy =
+                (unsigned long long)llrint((double)(-gy[j] * wx[j][a]) * sy_);
+            const size_t row = (size_t)wrapi(cx[j] - 1 + a, N) * N;
+            if (inx)
+                atomicAdd(&winy[((ax + a) * kAdjTY + ly) * TZ + lz], vy);
+            else
+                atomicAdd(AyI + (row + qy) * N + qz, vy);
+#pragma unroll
+            for (int b = 0; b < 3; b++) {
+                const unsigned long long vz =
+                    (unsigned long long)llrint((double)(-gz[j] * wx[j][a] * wy[j][b]) * sz_);
+                if (in)
+                    atomicAdd(&winz[((ax + a) * WX + ay + b) * TZ + lz], vz);
+                else
+                    atomicAdd(AzI + (row + wrapi(cy[j] - 1 + b, N)) * N + qz, vz);
+            }
+        }
     }
-    Ax[p] = -gx;
+    __syncthreads();
+    // 16 lanes a row; cells past the grid's z edge hold nothing
+    for (int r = threadIdx.x >> 4; r < WX * WX; r += 32) {
+        const unsigned long long v = winz[r * TZ + lz];
+        if (v)
+            atomicAdd(AzI + ((size_t)wrapi(wx0 + r / WX, N) * N + wrapi(wy0 + r % WX, N)) * N + qz,
+                      v);
+    }
+    for (int r = threadIdx.x >> 4; r < WX * kAdjTY; r += 32) {
+        const unsigned long long v = winy[r * TZ + lz];
+        if (v)
+            atomicAdd(AyI + ((size_t)wrapi(wx0 + r / kAdjTY, N) * N + y0 + r % kAdjTY) * N + qz, v);
+    }
 }
 
 template <typename T>
 __global__ void k_adj_fixed_to_real(const unsigned long long* __restrict__ I,
-                                    const unsigned long long* __restrict__ gmax, int which, T* A,
+                                    const double* __restrict__ gmax, int which, T* A,
                                     long n) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const double m = __longlong_as_double((long long)gmax[which]);
+    const double m = gmax[which];
     A[i] = (T)((double)(long long)I[i] * ldexp(m, -kAdjFixedBits));
 }
 
@@ -366,19 +512,23 @@ static int backward(Pipe<T>* P, const mitos_ic_config& cfg, const cx<T>* noise,
     T* Ax = reinterpret_cast<T*>(P->b(1));
     T* Ay = reinterpret_cast<T*>(P->b(2));
     T* Az = reinterpret_cast<T*>(P->a(1));
-    if (!P->adj_ws) MITOS_HIP_CHECK(hipMalloc(&P->adj_ws, sizeof(unsigned long long) *
-                                                          (2 * (size_t)n3 + 2)));
+    const unsigned tiles = adj_tiles(N);
+    if (!P->adj_ws)
+        MITOS_HIP_CHECK(hipMalloc(&P->adj_ws,
+                                  sizeof(unsigned long long) * (2 * (size_t)n3 + 2 + 2 * tiles)));
     unsigned long long* AyI = P->adj_ws;
     unsigned long long* AzI = AyI + n3;
-    unsigned long long* gmax = AzI + n3;
-    hipLaunchKernelGGL((k_fill<unsigned long long>), dim3(nblk(2 * n3 + 2)), dim3(256), 0, s,
-                       AyI, 2 * n3 + 2, 0ULL);
-    hipLaunchKernelGGL((k_adj_particles<T, 0>), dim3(nblk(n3)), dim3(256), 0, s, P->psi(0),
-                       P->psi(1), P->psi(2), (unsigned)P->prs(), grho, Ax, AyI, AzI, gmax, N, L,
-                       (float)L / N);
-    hipLaunchKernelGGL((k_adj_particles<T, 1>), dim3(nblk(n3)), dim3(256), 0, s, P->psi(0),
-                       P->psi(1), P->psi(2), (unsigned)P->prs(), grho, Ax, AyI, AzI, gmax, N, L,
-                       (float)L / N);
+    double* gmax = reinterpret_cast<double*>(AzI + n3);
+    double* part = gmax + 2;
+    T* gy = reinterpret_cast<T*>(P->a(0));
+    T* gz = reinterpret_cast<T*>(P->a(2));
+    hipLaunchKernelGGL((k_fill<unsigned long long>), dim3(nblk(2 * n3)), dim3(256), 0, s, AyI,
+                       2 * n3, 0ULL);
+    hipLaunchKernelGGL((k_adj_gradients<T>), dim3(tiles), dim3(256), 0, s, P->psi(0), P->psi(1),
+                       P->psi(2), (unsigned)P->prs(), grho, Ax, gy, gz, part, N, L, (float)L / N);
+    hipLaunchKernelGGL(k_adj_max, dim3(1), dim3(1024), 0, s, part, tiles, gmax);
+    hipLaunchKernelGGL((k_adj_scatter<T>), dim3(tiles), dim3(512), 0, s, P->psi(0), P->psi(1),
+                       (unsigned)P->prs(), gy, gz, AyI, AzI, gmax, N, L, (float)L / N);
     hipLaunchKernelGGL((k_adj_fixed_to_real<T>), dim3(nblk(n3)), dim3(256), 0, s, AyI, gmax, 0,
                        Ay, n3);
     hipLaunchKernelGGL((k_adj_fixed_to_real<T>), dim3(nblk(n3)), dim3(256), 0, s, AzI, gmax, 1,

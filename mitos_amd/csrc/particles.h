@@ -1045,8 +1045,10 @@ __global__ void __launch_bounds__(TXN / PP * TY * TZ) __attribute__((amdgpu_wave
 // analyse/src/mitos_read.c:285-320: base cell and the eight CIC weights of a
 // particle, the weights as 2^-40 fixed point in the reference's corner order
 // (000, 100, 010, 001, 110, 101, 011, 111).
-__device__ __forceinline__ void cic_cell(float X, float Y, float Z, int N, double boxlen, int& iX,
-                                         int& iY, int& iZ, double& dx, double& dy, double& dz) {
+// (P: float, the particle arrays; double, the positions of the FP64 adjoint)
+template <typename P>
+__device__ __forceinline__ void cic_cell(P X, P Y, P Z, int N, double boxlen, int& iX, int& iY,
+                                         int& iZ, double& dx, double& dy, double& dz) {
 #pragma clang fp contract(off)
     const double cell = boxlen / N;
     const double Xc = fwrap_fast((double)X, boxlen) / cell;
@@ -1217,9 +1219,56 @@ __device__ __forceinline__ void cic_cell_t(T x, T icell, int N, int& i, T& d) {
     }
 }
 
-// Adjoint-mode particles: moves in T, positions kept in T for the deposit
-// (their float copies go to X/Y/Z), fixed-point weights 2^-shift with global
-// atomics (order independent).
+// Lattice site of thread t's particle j in the order of the adjoint's particle
+// kernels: work-groups of 256 threads over 8 x 8 x 16 tiles (x, y, z), four
+// particles a thread, so the taps of a work-group share lines in L1.  False
+// past the grid's edge (N = 8, 24).
+constexpr int kAdjTX = 8, kAdjTY = 8, kAdjTZ = 16;
+inline unsigned adj_tiles(int N) {
+    return (unsigned)((N / kAdjTX) * (N / kAdjTY) * ((N + kAdjTZ - 1) / kAdjTZ));
+}
+__device__ __forceinline__ void adj_tile(unsigned b, int N, int& x0, int& y0, int& z0) {
+    const unsigned ntz = (unsigned)(N + kAdjTZ - 1) / kAdjTZ, nty = (unsigned)N / kAdjTY;
+    z0 = (int)(b % ntz) * kAdjTZ;
+    y0 = (int)(b / ntz % nty) * kAdjTY;
+    x0 = (int)(b / (ntz * nty)) * kAdjTX;
+}
+
+// The adjoint's FP64 moves: positions in T (dense N^3 arrays) and their float
+// copies.
+template <typename T>
+__global__ void __launch_bounds__(256)
+    k_moves_s(const T* __restrict__ sx, const T* __restrict__ sy, const T* __restrict__ sz,
+              unsigned rs, int N, double boxlen, float spacing, float* __restrict__ X,
+              float* __restrict__ Y, float* __restrict__ Z, T* __restrict__ xt,
+              T* __restrict__ yt, T* __restrict__ zt) {
+    int x0, y0, z0;
+    adj_tile(xcd_block(blockIdx.x, gridDim.x), N, x0, y0, z0);
+    const int qz = z0 + (threadIdx.x & 15), qy = y0 + ((threadIdx.x >> 4) & 7);
+    if (qz >= N) return;
+    const T L = (T)boxlen, sN = (T)(N / boxlen);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int qx = x0 + (int)(threadIdx.x >> 7) + 2 * j;
+        T x, y, z;
+        moves_s(sx, sy, sz, rs, N, sN, spacing, qx, qy, qz, x, y, z);
+        x = wrap_pos(x, L);
+        y = wrap_pos(y, L);
+        z = wrap_pos(z, L);
+        const size_t p = ((size_t)qx * N + qy) * N + qz;
+        X[p] = (float)x;
+        Y[p] = (float)y;
+        Z[p] = (float)z;
+        xt[p] = x;
+        yt[p] = y;
+        zt[p] = z;
+    }
+}
+
+// The adjoint's FP64 moves and deposit on grids without deposit tiles (N not a
+// multiple of 32): positions kept in T for the deposit (their float copies go
+// to X/Y/Z), fixed-point weights 2^-shift with global atomics (order
+// independent).
 template <typename T>
 __global__ void __launch_bounds__(256)
     k_move_deposit_s(const T* __restrict__ sx, const T* __restrict__ sy,
@@ -1305,8 +1354,8 @@ __device__ __forceinline__ void cic_axis_f(float x, float cell, float cinv, int 
 // for the tiled deposit: base cell q + r with r the periodic cell offset in
 // [-N/2, N/2) (so the base index lies in [-N/2, 3N/2)), and the in-cell
 // offsets.
-template <typename W>
-__device__ __forceinline__ void cic_lattice_cell(float x, float y, float z, int N, double boxlen,
+template <typename W, typename P>
+__device__ __forceinline__ void cic_lattice_cell(P x, P y, P z, int N, double boxlen,
                                                  float cell, float cinv, int qx, int qy, int qz,
                                                  int& rx, int& ry, int& rz, W& fx, W& fy,
                                                  W& fz) {
@@ -1404,11 +1453,12 @@ __device__ __noinline__ inline void cic_list_carry(const CicLists& l, unsigned m
 // W = double: the reference's double weights in units of 2^-40 (FP64
 // pipeline), 64-bit window; W = float: float weights in units of 2^-24 (FP32
 // pipeline), 32-bit window with carries.
+// PT: type of the positions (double: the FP64 adjoint's)
 template <typename W, int PX, int PY, int PZ, int RX, int RY, int RZ, int NT,
-          bool STREAM = false>
+          bool STREAM = false, typename PT = float>
 __global__ void __launch_bounds__(NT)
-    k_cic_lattice(const float* __restrict__ X, const float* __restrict__ Y,
-                  const float* __restrict__ Z, int N, double boxlen, unsigned long long* grid,
+    k_cic_lattice(const PT* __restrict__ X, const PT* __restrict__ Y,
+                  const PT* __restrict__ Z, int N, double boxlen, unsigned long long* grid,
                   int ntiles, typename CicWin<W>::type* __restrict__ scratch = nullptr,
                   int* __restrict__ means = nullptr, int* __restrict__ mmax = nullptr,
                   CicLists lists = CicLists{}) {
@@ -1432,7 +1482,7 @@ __global__ void __launch_bounds__(NT)
     for (int c = threadIdx.x; c < R; c += NT) win[c] = 0;
     if (threadIdx.x == 0) qn = 0;
     // positions of the group's first tile
-    float px[K], py[K], pz[K];
+    PT px[K], py[K], pz[K];
     auto load = [&](int tile) {
         const int tz = tile % ntz, ty = (tile / ntz) % nty, tx = tile / (ntz * nty);
 #pragma unroll
@@ -1753,9 +1803,9 @@ __global__ void __launch_bounds__(256)
 }
 
 // the tile kernel of window type W
-template <typename W, bool STREAM = false, typename C = CicTile<W>>
+template <typename W, bool STREAM = false, typename PT = float, typename C = CicTile<W>>
 constexpr auto cic_lattice_kernel() {
-    return k_cic_lattice<W, C::PX, C::PY, C::PZ, C::RX, C::RY, C::RZ, C::NT, STREAM>;
+    return k_cic_lattice<W, C::PX, C::PY, C::PZ, C::RX, C::RY, C::RZ, C::NT, STREAM, PT>;
 }
 
 static __global__ void k_zero_i32(int* p, int n) {
@@ -1813,8 +1863,8 @@ inline CicLists cic_lists(int N, void* ws, void* lists_mem) {
 // the windows go to ws, far particles and carries to the lists, and
 // cic_gather_launch then cic_far_launch write the grid, which need not be
 // cleared.  Otherwise the windows are added to a cleared grid with atomics.
-template <typename W, bool STREAM>
-inline int cic_lattice_launch(const float* X, const float* Y, const float* Z, int N,
+template <typename W, bool STREAM, typename PT = float>
+inline int cic_lattice_launch(const PT* X, const PT* Y, const PT* Z, int N,
                               double boxlen, unsigned long long* grid, void* ws,
                               void* lists_mem, hipStream_t s) {
     typedef CicTile<W> C;
@@ -1834,7 +1884,7 @@ inline int cic_lattice_launch(const float* X, const float* Y, const float* Z, in
             MITOS_HIP_CHECK(
                 hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
             MITOS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per, cic_lattice_kernel<W, STREAM>(), C::NT, 0));
+                &per, cic_lattice_kernel<W, STREAM, PT>(), C::NT, 0));
             if (cus <= 0 || per <= 0) return MITOS_ERR_DEVICE;
             it = resident.emplace(dev, cus * per).first;
         }
@@ -1853,7 +1903,7 @@ inline int cic_lattice_launch(const float* X, const float* Y, const float* Z, in
         // mean-offset maxima (meta[0..2]) and list counts (meta[4..5]) start at 0
         hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, meta, 8);
     }
-    hipLaunchKernelGGL((cic_lattice_kernel<W, STREAM>()), dim3(groups), dim3(C::NT), 0, s, X, Y,
+    hipLaunchKernelGGL((cic_lattice_kernel<W, STREAM, PT>()), dim3(groups), dim3(C::NT), 0, s, X, Y,
                        Z, N, boxlen, grid, ntiles, scratch, means, meta, lists);
     return MITOS_OK;
 }
