@@ -89,6 +89,17 @@ int kspec_from_callback(void (*compute)(struct kernel*), const void* params, int
     return MITOS_OK;
 }
 
+template <int HOW, typename TW, typename TR>
+int launch_apply(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double boxlen,
+                 const KSpec& ks, const double* tab, const TransferTab& t = TransferTab{}) {
+    const long n = nx * N * (N / 2 + 1);
+    if (n <= 0) return api_sync();
+    hipLaunchKernelGGL((k_apply_kernel<TW, TR, HOW>), dim3(nblk(n, kApplyBlock)), dim3(256), 0,
+                       api_stream(), w, r, N, x0, nx, boxlen, ks, tab, t);
+    MITOS_TRY(launch_status());
+    return api_sync();
+}
+
 // kernel_(inv_)transfer_function: the k vector and the selected function's
 // two time rows go to the device, the modes are evaluated there
 template <typename TW, typename TR>
@@ -106,11 +117,7 @@ int apply_transfer(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double b
     MITOS_HIP_CHECK(copy_sync(d, pt->k, sizeof(double) * ks, hipMemcpyHostToDevice));
     MITOS_HIP_CHECK(copy_sync(d + ks, rows, sizeof(double) * 2 * ks, hipMemcpyHostToDevice));
     TransferTab t{d, d + ks, d + 2 * ks, ks, sp->u_tau, invert};
-    const long n = nx * N * (N / 2 + 1);
-    hipLaunchKernelGGL((k_apply_transfer<TW, TR>), dim3(nblk(n)), dim3(256), 0, api_stream(), w,
-                       r, N, (long)(N / 2 + 1), x0, nx, boxlen, t);
-    MITOS_TRY(launch_status());
-    return api_sync();
+    return launch_apply<APPLY_TRANSFER>(w, r, N, x0, nx, boxlen, KSpec{}, nullptr, t);
 }
 
 // Any other callback: evaluated on the host for every mode with the
@@ -200,11 +207,25 @@ int apply_kernel(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double box
     if (kr == MITOS_ERR_UNSUPPORTED)
         return apply_kernel_host<TW, TR>(w, r, N, x0, nx, boxlen, compute, params);
     MITOS_TRY(kr);
-    const long n = nx * N * (N / 2 + 1);
-    hipLaunchKernelGGL((k_apply_kernel<TW, TR>), dim3(nblk(n)), dim3(256), 0, api_stream(), w,
-                       r, N, (long)(N / 2 + 1), x0, nx, boxlen, ks);
-    MITOS_TRY(launch_status());
-    return api_sync();
+    // tables of a window's N factors, and of the spectra's powers and logarithms
+    // over n^2 from 64^3 on, where the grid has 21 modes and more per entry
+    if (ks.id == KID_UNDO_WINDOW) {
+        double* tab = (double*)workspace(9, sizeof(double) * N);
+        if (!tab) return MITOS_ERR_ALLOC;
+        hipLaunchKernelGGL(k_window_factors, dim3(nblk(N)), dim3(256), 0, api_stream(), ks, N,
+                           boxlen, tab);
+        return launch_apply<APPLY_WINDOW>(w, r, N, x0, nx, boxlen, ks, tab);
+    }
+    if (N >= 64 && (ks.id == KID_POWER_NO_TRANSFER || ks.id == KID_SQRT_POWER_LAW ||
+                    ks.id == KID_BBKS)) {
+        const long n2 = 3L * (N / 2) * (N / 2) + 1;
+        double* tab = (double*)workspace(9, sizeof(double) * n2);
+        if (!tab) return MITOS_ERR_ALLOC;
+        hipLaunchKernelGGL(k_radial_values, dim3(nblk(n2)), dim3(256), 0, api_stream(), ks, n2,
+                           boxlen, tab);
+        return launch_apply<APPLY_RADIAL>(w, r, N, x0, nx, boxlen, ks, tab);
+    }
+    return launch_apply<APPLY_DIRECT>(w, r, N, x0, nx, boxlen, ks, nullptr);
 }
 
 template <typename T>
