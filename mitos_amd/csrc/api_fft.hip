@@ -236,26 +236,50 @@ int scale_complex(cx<T>* a, long n, double s) {
     return api_sync();
 }
 
+// Two work grids of the transforms, or one used twice where two do not fit
+template <typename T>
+bool work_grids(int N, cx<T>** w1, cx<T>** w2) {
+    const size_t bytes = work_grid_bytes<T>(N);
+    if ((*w1 = (cx<T>*)workspace(0, 2 * bytes))) {
+        *w2 = *w1 + bytes / sizeof(cx<T>);
+        return true;
+    }
+    (void)hipGetLastError();
+    *w2 = *w1 = (cx<T>*)workspace(0, bytes);
+    return *w1 != nullptr;
+}
+
+// r2c of an N^3 array with row stride rs into the (N, N, N/2+1) layout, times
+// scale, issued on the library stream
+template <typename T, typename OPX>
+int r2c_issue(int N, const T* in, long rs, cx<T>* out, OPX ox) {
+    if (!in || !out) return MITOS_ERR_ARG;
+    if (!size_supported(N)) return MITOS_ERR_UNSUPPORTED;
+    cx<T>*w1, *w2;
+    if (!work_grids(N, &w1, &w2)) return MITOS_ERR_ALLOC;
+    RealRowLoader<T> ld{in, rs, 0};
+    return r2c_3d<T>(N, ld, w1, w2, out, N / 2 + 1, ox, api_stream());
+}
+
+template <typename T>
+int c2r_issue(int N, const cx<T>* in, T* out, long rs, double scale) {
+    if (!in || !out) return MITOS_ERR_ARG;
+    if (!size_supported(N)) return MITOS_ERR_UNSUPPORTED;
+    cx<T>*w1, *w2;
+    if (!work_grids(N, &w1, &w2)) return MITOS_ERR_ALLOC;
+    return c2r_3d<T>(N, in, N / 2 + 1, w1, w2, out, rs, (T)scale, OpNone(), api_stream());
+}
+
 // unnormalised r2c of an N^3 array with row stride rs into the (N, N, N/2+1) layout
 template <typename T>
 int r2c_plain(int N, const T* in, long rs, cx<T>* out) {
-    if (!in || !out) return MITOS_ERR_ARG;
-    if (!size_supported(N)) return MITOS_ERR_UNSUPPORTED;
-    GridLayout g{N, N / 2 + 1, rs};
-    RealRowLoader<T> ld{in, rs, 0};
-    MITOS_TRY((r2c_3d<T>(ld, out, g, 1, 0, OpNone(), OpNone(), OpNone(), api_stream())));
+    MITOS_TRY((r2c_issue<T>(N, in, rs, out, OpNone())));
     return api_sync();
 }
 
 template <typename T>
 int c2r_plain(int N, const cx<T>* in, T* out, long rs, double scale) {
-    if (!in || !out) return MITOS_ERR_ARG;
-    if (!size_supported(N)) return MITOS_ERR_UNSUPPORTED;
-    GridLayout g{N, N / 2 + 1, rs};
-    cx<T>* ws = (cx<T>*)workspace(0, sizeof(cx<T>) * half_elems(N));
-    if (!ws) return MITOS_ERR_ALLOC;
-    MITOS_TRY((c2r_3d<T>(in, ws, out, g, 1, 0, 0, (T)scale, OpNone(), OpNone(), OpNone(),
-                         api_stream())));
+    MITOS_TRY(c2r_issue<T>(N, in, out, rs, scale));
     return api_sync();
 }
 
@@ -417,11 +441,9 @@ extern "C" int fft_r2c_dg(struct distributed_grid* dg) {
     if (!size_supported(N)) return set_last_error(MITOS_ERR_UNSUPPORTED);
     const double boxvol = dg->boxlen * dg->boxlen * dg->boxlen;
     const double s = boxvol / ((long long)N * N * N);
-    GridLayout g{N, N / 2 + 1, N + 2};
-    RealRowLoader<double> ld{dg->box, N + 2, 0};
-    cx<double>* out = reinterpret_cast<cx<double>*>(dg->fbox);
-    MITOS_TRY(set_last_error(r2c_3d<double>(ld, out, g, 1, 0, OpNone(), OpNone(),
-                                            OpScale<double>{s}, api_stream())));
+    MITOS_TRY(set_last_error(r2c_issue<double>(N, dg->box, N + 2,
+                                               reinterpret_cast<cx<double>*>(dg->fbox),
+                                               OpScale<double>{s})));
     dg->momentum_space = 1;
     return set_last_error(api_sync());
 }

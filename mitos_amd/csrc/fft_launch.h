@@ -111,97 +111,11 @@ struct OuterPerBlock {
     static constexpr int value = (AXIS == 0 && L >= 64) ? 2 : 1;
 };
 
-template <typename T, int L, int C, int AXIS, int DIR, bool SPLIT, typename OP, typename RAD>
-struct StridedK;
-template <typename T, int L, int C, int AXIS, int DIR, bool SPLIT, typename OP, int... Rs>
-struct StridedK<T, L, C, AXIS, DIR, SPLIT, OP, Radices<Rs...>> {
-    static void go(dim3 g, dim3 b, hipStream_t s, const cx<T>* in, cx<T>* out, long hs,
-                   int ncols, long bstride, const cx<T>* tw, OP op) {
-        hipLaunchKernelGGL((k_pass_strided<T, L, LineCfg<L>::E, C, AXIS, DIR, SPLIT,
-                                           OuterPerBlock<L, AXIS>::value, OP, Rs...>),
-                           g, b, 0, s, in, out, hs, ncols, bstride, tw, op, 0);
-    }
-};
-
-template <typename T, int L, int AXIS, int DIR, typename OP>
-int strided_pass(const cx<T>* in, cx<T>* out, long hs, int nbatch, long bstride, OP op,
-                 hipStream_t s) {
-    constexpr int C = ColTile<T>::C;
-    constexpr int E = LineCfg<L>::E;
-    constexpr int TPL = L / E;
-    constexpr bool SPLIT = 2 * LdsMap<T, L, C, true>::SIZE * sizeof(T) > 81920;
-    const int ncols = L / 2 + 1;
-    if (!strided_offsets_fit<T, L, AXIS>(TPL, hs)) return MITOS_ERR_UNSUPPORTED;
-    const cx<T>* tw = twiddles<T>(L);
-    if (!tw) return MITOS_ERR_ALLOC;
-    dim3 grid((stored_cols<T, C>(ncols, hs) + C - 1) / C, L / OuterPerBlock<L, AXIS>::value,
-              nbatch);
-    StridedK<T, L, C, AXIS, DIR, SPLIT, OP, typename LineCfg<L>::R>::go(
-        grid, dim3(TPL * C), s, in, out, hs, ncols, bstride, tw, op);
-    return launch_status();
-}
-
 // ---- z passes ----------------------------------------------------------------
 template <int TPL>
 struct RowsPerBlock {
     static constexpr int value = TPL >= 256 ? 1 : 256 / TPL;
 };
-
-template <typename T, int L, int RW, int HO, typename OP, typename RAD>
-struct ZC2RK;
-template <typename T, int L, int RW, int HO, typename OP, int... Rs>
-struct ZC2RK<T, L, RW, HO, OP, Radices<Rs...>> {
-    template <typename... A>
-    static void go(dim3 g, dim3 b, hipStream_t s, A... a) {
-        hipLaunchKernelGGL((k_zc2r<T, L, LineCfg<L>::E, RW, HO, OP, Rs...>), g, b, 0, s, a...);
-    }
-};
-
-// HO > 0 writes rows with a periodic one-value halo (see k_zc2r)
-template <typename T, int N, typename OP, int HO = 0>
-int zc2r_pass(const cx<T>* in, T* out, long hs, long rs, int nbatch, long inb, long outb,
-              T scale, OP op, hipStream_t s) {
-    if (rs < N + (HO > 0 ? HO + 1 : 0)) return MITOS_ERR_ARG;
-    constexpr int L = N / 2;
-    constexpr int TPL = L / LineCfg<L>::E;
-    constexpr int RW = RowsPerBlock<TPL>::value;
-    const long nrows = (long)N * N;
-    const cx<T>* tw = twiddles<T>(L);
-    const cx<T>* twN = twiddles<T>(N);
-    if (!tw || !twN) return MITOS_ERR_ALLOC;
-    dim3 grid((unsigned)((nrows + RW - 1) / RW), nbatch);
-    ZC2RK<T, L, RW, HO, OP, typename LineCfg<L>::R>::go(grid, dim3(TPL * RW), s, in, out, 0L,
-                                                     nrows, N, hs, rs, inb, outb, tw, twN, scale,
-                                                     op);
-    return launch_status();
-}
-
-template <typename T, int L, int RW, typename LOADER, typename OP, typename RAD>
-struct ZR2CK;
-template <typename T, int L, int RW, typename LOADER, typename OP, int... Rs>
-struct ZR2CK<T, L, RW, LOADER, OP, Radices<Rs...>> {
-    template <typename... A>
-    static void go(dim3 g, dim3 b, hipStream_t s, A... a) {
-        hipLaunchKernelGGL((k_zr2c<T, L, LineCfg<L>::E, RW, LOADER, OP, Rs...>), g, b, 0, s,
-                           a...);
-    }
-};
-
-template <typename T, int N, typename LOADER, typename OP>
-int zr2c_pass(LOADER loader, cx<T>* out, long hs, int nbatch, long outb, OP op, hipStream_t s) {
-    constexpr int L = N / 2;
-    constexpr int TPL = L / LineCfg<L>::E;
-    constexpr int RW = RowsPerBlock<TPL>::value;
-    const long nrows = (long)N * N;
-    const cx<T>* tw = twiddles<T>(L);
-    const cx<T>* twN = twiddles<T>(N);
-    if (!tw || !twN) return MITOS_ERR_ALLOC;
-    dim3 grid((unsigned)((nrows + RW - 1) / RW), nbatch);
-    ZR2CK<T, L, RW, LOADER, OP, typename LineCfg<L>::R>::go(grid, dim3(TPL * RW), s, loader,
-                                                             out, 0L, nrows, N, hs, outb, tw, twN,
-                                                             op);
-    return launch_status();
-}
 
 // ---- tunable schedules ---------------------------------------------------------
 // Variants of the plain passes that the autotuner (autotune.h) times on the
@@ -254,23 +168,24 @@ template <typename T, int L, int C, int AXIS, int DIR, bool SPLIT, typename OP, 
           int... Rs>
 struct StridedKV<T, L, C, AXIS, DIR, SPLIT, OP, CFG, Radices<Rs...>> {
     static void go(dim3 g, dim3 b, hipStream_t s, const cx<T>* in, cx<T>* out, long hs,
-                   int ncols, long bstride, const cx<T>* tw, OP op, int o0) {
+                   long ohs, int ncols, const cx<T>* tw, OP op, int o0) {
         hipLaunchKernelGGL((k_pass_strided<T, L, CFG::E, C, AXIS, DIR, SPLIT,
                                            OuterPerBlock<L, AXIS>::value, OP, Rs...>),
-                           g, b, 0, s, in, out, hs, ncols, bstride, tw, op, o0);
+                           g, b, 0, s, in, out, hs, ohs, ncols, tw, op, o0);
     }
 };
 
-// outer indices o0 .. o0+no-1 only when no > 0
+// in: rows of hs, out: rows of ohs; outer indices o0 .. o0+no-1 only when no > 0
 template <typename T, int L, int AXIS, int DIR, int V, typename OP>
-int strided_pass_v(const cx<T>* in, cx<T>* out, long hs, int nbatch, long bstride, OP op,
-                   hipStream_t s, int o0 = 0, int no = 0) {
+int strided_pass_v(const cx<T>* in, long hs, cx<T>* out, long ohs, OP op, hipStream_t s,
+                   int o0 = 0, int no = 0) {
     if (no <= 0) {
         o0 = 0;
         no = L;
     }
     constexpr int KO = OuterPerBlock<L, AXIS>::value;
     if (o0 < 0 || o0 + no > L || o0 % KO || no % KO) return MITOS_ERR_ARG;
+    if (in == out && hs != ohs) return MITOS_ERR_ARG;
     typedef StridedSched<T, L, V> S;
     constexpr int C = S::C;
     constexpr long LDS2 = 2 * (long)LdsMap<T, L, C, true>::SIZE * (long)sizeof(T);
@@ -279,25 +194,20 @@ int strided_pass_v(const cx<T>* in, cx<T>* out, long hs, int nbatch, long bstrid
     if (!strided_offsets_fit<T, L, AXIS>(S::TPL, hs)) return MITOS_ERR_UNSUPPORTED;
     const cx<T>* tw = twiddles<T>(L);
     if (!tw) return MITOS_ERR_ALLOC;
-    dim3 grid((stored_cols<T, C>(ncols, hs) + C - 1) / C, no / KO, nbatch);
+    dim3 grid((stored_cols<T, C>(ncols, ohs) + C - 1) / C, no / KO);
     StridedKV<T, L, C, AXIS, DIR, SPLIT, OP, typename S::CFG>::go(
-        grid, dim3(S::TPL * C), s, in, out, hs, ncols, bstride, tw, op, o0);
+        grid, dim3(S::TPL * C), s, in, out, hs, ohs, ncols, tw, op, o0);
     return launch_status();
 }
 
 // strided pass with a run-time schedule variant
 template <typename T, int L, int AXIS, int DIR, typename OP>
-int strided_pass_tuned(int variant, const cx<T>* in, cx<T>* out, long hs, int nbatch,
-                       long bstride, OP op, hipStream_t s, int o0 = 0, int no = 0) {
+int strided_pass_tuned(int variant, const cx<T>* in, cx<T>* out, long hs, OP op, hipStream_t s) {
     switch (variant) {
-        case 1:
-            return strided_pass_v<T, L, AXIS, DIR, 1>(in, out, hs, nbatch, bstride, op, s, o0, no);
-        case 2:
-            return strided_pass_v<T, L, AXIS, DIR, 2>(in, out, hs, nbatch, bstride, op, s, o0, no);
-        case 3:
-            return strided_pass_v<T, L, AXIS, DIR, 3>(in, out, hs, nbatch, bstride, op, s, o0, no);
-        default:
-            return strided_pass_v<T, L, AXIS, DIR, 0>(in, out, hs, nbatch, bstride, op, s, o0, no);
+        case 1: return strided_pass_v<T, L, AXIS, DIR, 1>(in, hs, out, hs, op, s);
+        case 2: return strided_pass_v<T, L, AXIS, DIR, 2>(in, hs, out, hs, op, s);
+        case 3: return strided_pass_v<T, L, AXIS, DIR, 3>(in, hs, out, hs, op, s);
+        default: return strided_pass_v<T, L, AXIS, DIR, 0>(in, hs, out, hs, op, s);
     }
 }
 
@@ -414,25 +324,49 @@ int zr2c_pass_tuned(int variant, LOADER loader, cx<T>* out, long hs, int nbatch,
 }
 
 // ---- composed 3D transforms ---------------------------------------------------
-// c2r: x (in -> ws), y (ws -> ws), z (ws -> out).  The input is left unchanged.
-template <typename T, typename OPX, typename OPY, typename OPZ>
-int c2r_3d(const cx<T>* in, cx<T>* ws, T* out, const GridLayout& g, int nb, long cb, long rb,
-           T scale, OPX ox, OPY oy, OPZ oz, hipStream_t s) {
-    return with_size(g.N, [&]<int NN>() -> int {
-        MITOS_TRY((strided_pass<T, NN, 0, 1>(in, ws, g.hs, nb, cb, ox, s)));
-        MITOS_TRY((strided_pass<T, NN, 1, 1>(ws, ws, g.hs, nb, cb, oy, s)));
-        return zc2r_pass<T, NN>(ws, out, g.hs, g.rs, nb, cb, rb, scale, oz, s);
+// The passes between the caller's arrays run through two work grids w1, w2 of
+// whole 128-byte rows (work_row elements), out of place: a pass over the dense
+// rows of N/2+1 values splits every tile row over two lines, and one in place
+// streams slower.  The pass at the caller's dense grid is the y pass, whose tiles
+// of one plane meet in L2 (512^3 FP64: 0.44 ms reading and 0.49 ms writing it, an
+// x pass 0.54 and 0.64 ms).  Whole transforms at 512^3 in FP64, against in-place
+// passes over dense rows: c2r 1.58 -> 1.31 ms, r2c 1.61 -> 1.36 ms, bound by HBM
+// (three passes of 2.15 GB at 4.8 TB/s).  w2 == w1 transforms in place.  Schedules: variant 0 of the strided passes, variant 1 of
+// the z passes, which measured within 3% of the fastest at every size but FP64
+// 768^3 r2c (the 16 values per thread of variant 0 take twice as long in FP64 at
+// 256^3 and 512^3: r2c 907 against 424 us).
+template <typename T>
+inline long work_row(int N) {
+    const long q = 128 / (long)sizeof(cx<T>);
+    return (N / 2 + 1 + q - 1) / q * q;
+}
+template <typename T>
+inline size_t work_grid_bytes(int N) {
+    return sizeof(cx<T>) * (size_t)N * N * (size_t)work_row<T>(N);
+}
+
+// c2r: y (in -> w1, values through op.pre), x (w1 -> w2), z (w2 -> out).  The
+// input is left unchanged (unless it is w1).
+template <typename T, typename OP>
+int c2r_3d(int N, const cx<T>* in, long ihs, cx<T>* w1, cx<T>* w2, T* out, long rs, T scale,
+           OP op, hipStream_t s) {
+    const long hs = work_row<T>(N);
+    return with_size(N, [&]<int NN>() -> int {
+        MITOS_TRY((strided_pass_v<T, NN, 1, 1, 0>(in, ihs, w1, hs, op, s)));
+        MITOS_TRY((strided_pass_v<T, NN, 0, 1, 0>(w1, hs, w2, hs, OpNone(), s)));
+        return zc2r_pass_v<T, NN, 1, 0>(w2, out, hs, rs, 1, 0, 0, scale, OpNone(), s);
     });
 }
 
-// r2c: z (loader -> out), y (out -> out), x (out -> out).
-template <typename T, typename LOADER, typename OPZ, typename OPY, typename OPX>
-int r2c_3d(LOADER loader, cx<T>* out, const GridLayout& g, int nb, long cb, OPZ oz, OPY oy,
-           OPX ox, hipStream_t s) {
-    return with_size(g.N, [&]<int NN>() -> int {
-        MITOS_TRY((zr2c_pass<T, NN>(loader, out, g.hs, nb, cb, oz, s)));
-        MITOS_TRY((strided_pass<T, NN, 1, -1>(out, out, g.hs, nb, cb, oy, s)));
-        return strided_pass<T, NN, 0, -1>(out, out, g.hs, nb, cb, ox, s);
+// r2c: z (loader -> w1), x (w1 -> w2), y (w2 -> out, values through op.post).
+template <typename T, typename LOADER, typename OP>
+int r2c_3d(int N, LOADER loader, cx<T>* w1, cx<T>* w2, cx<T>* out, long ohs, OP op,
+           hipStream_t s) {
+    const long hs = work_row<T>(N);
+    return with_size(N, [&]<int NN>() -> int {
+        MITOS_TRY((zr2c_pass_v<T, NN, 1>(loader, w1, hs, 1, 0, OpNone(), s)));
+        MITOS_TRY((strided_pass_v<T, NN, 0, -1, 0>(w1, hs, w2, hs, OpNone(), s)));
+        return strided_pass_v<T, NN, 1, -1, 0>(w2, hs, out, ohs, op, s);
     });
 }
 

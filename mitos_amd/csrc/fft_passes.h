@@ -106,13 +106,13 @@ __host__ __device__ __forceinline__ int stored_cols(int ncols, long hs) {
 // AXIS 0: lines along x, outer index o = y;  AXIS 1: lines along y, o = x.
 // Work-group (bx, by) transforms column tile bx for the KO outer indices
 // o = o0 + by*KO + i, i < KO (consecutive y rows of an x pass stream faster
-// from one work-group than from KO); blockIdx.z selects one of several grids
-// spaced `batch_stride` apart.  in == out is allowed: every thread stores
-// exactly the elements it loaded.
+// from one work-group than from KO).  hs, ohs: row strides of in and out.
+// in == out is allowed (hs == ohs): every thread stores exactly the elements it
+// loaded.
 template <typename T, int L, int E, int C, int AXIS, int DIR, bool SPLIT, int KO, typename OP,
           int... Rs>
 __global__ void __launch_bounds__(L / E * C)
-    k_pass_strided(const cx<T>* in, cx<T>* out, long hs, int ncols, long batch_stride,
+    k_pass_strided(const cx<T>* in, cx<T>* out, long hs, long ohs, int ncols,
                    const cx<T>* __restrict__ tw, OP op, int o0) {
     constexpr int TPL = L / E;
     typedef LdsMap<T, L, C, true> M;
@@ -123,9 +123,11 @@ __global__ void __launch_bounds__(L / E * C)
     xcd_block2(bx, by);
     const int col = bx * C + c;
     const bool ok = col < ncols;
-    const bool wok = col < stored_cols<T, C>(ncols, hs);
+    const bool wok = col < stored_cols<T, C>(ncols, ohs);
     const long pstride = (AXIS == 0) ? (long)L * hs : hs;
     const long ostride = (AXIS == 0) ? hs : (long)L * hs;
+    const long wpstride = (AXIS == 0) ? (long)L * ohs : ohs;
+    const long wostride = (AXIS == 0) ? ohs : (long)L * ohs;
     // loads address a work-group-uniform base per element plus one 32-bit
     // per-thread offset (the launcher checks TPL * pstride elements fit in 32
     // bits): no 64-bit address registers per element
@@ -133,9 +135,8 @@ __global__ void __launch_bounds__(L / E * C)
 #pragma unroll 1
     for (int i = 0; i < KO; i++) {
         const int o = o0 + (int)by * KO + i;
-        const long base = blockIdx.z * batch_stride + (long)o * ostride + col;
-        const char* ub = reinterpret_cast<const char*>(in + blockIdx.z * batch_stride +
-                                                       (long)o * ostride + (long)bx * C);
+        const long base = (long)o * wostride + col;
+        const char* ub = reinterpret_cast<const char*>(in + (long)o * ostride + (long)bx * C);
         // per-row copies: LDS addresses and twiddles kept live across the rows
         // would take registers from the values
         int tl = t, cl = c;
@@ -159,7 +160,7 @@ __global__ void __launch_bounds__(L / E * C)
                 const int p = tl + TPL * e;
                 cx<T> a = !ok ? mk<T>(0, 0)
                               : (AXIS == 0) ? op.post(v[e], p, o, col) : op.post(v[e], o, p, col);
-                st(out + base + (long)p * pstride, a);
+                st(out + base + (long)p * wpstride, a);
             }
         }
     }

@@ -132,13 +132,4 @@ __device__ __forceinline__ void xcd_block2(unsigned& bx, unsigned& by) {
 // Signed frequency index of grid index i (src/fft.c:31-33: index N/2 -> +N/2).
 __host__ __device__ __forceinline__ int freq_index(int i, int N) { return (i > N / 2) ? i - N : i; }
 
-// Layout of one realization's grids in device memory.
-//   complex half grid: element (x, y, z') at (x*N + y)*hs + z', z' in [0, N/2]
-//   real grid:         element (x, y, z ) at (x*N + y)*rs + z , z  in [0, N)
-struct GridLayout {
-    int N;
-    long hs;  // complex row stride (elements), >= N/2+1
-    long rs;  // real row stride (elements), >= N
-};
-
 }  // namespace mitos

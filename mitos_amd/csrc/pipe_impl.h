@@ -123,12 +123,10 @@ int Pipe<T>::autotune(hipStream_t s) {
             for (int v = 0; v < kFftVariants; v++) {
                 // out of place, as the runs use them
                 MITOS_TRY(time_it([&] {
-                    return strided_pass_tuned<T, NN, 1, -1>(v, K, a(0), hs, 1, 0, OpNone(),
-                                                            s);
+                    return strided_pass_tuned<T, NN, 1, -1>(v, K, a(0), hs, OpNone(), s);
                 }, &sc.ms[TUNE_Y_FWD][v]));
                 MITOS_TRY(time_it([&] {
-                    return strided_pass_tuned<T, NN, 0, -1>(v, a(0), K, hs, 1, 0, OpNone(),
-                                                            s);
+                    return strided_pass_tuned<T, NN, 0, -1>(v, a(0), K, hs, OpNone(), s);
                 }, &sc.ms[TUNE_X_FWD][v]));
                 MITOS_TRY(time_it([&] {
                     // the displacement grids' layout of the default form
@@ -165,19 +163,16 @@ int Pipe<T>::fft_timing(hipStream_t s, int reps, float* r2c_ms, float* c2r_ms) {
     const int rc = with_size(N, [&]<int NN>() -> int {
         RealRowLoader<T> ld{real, rs, 0};
         auto r2c = [&]() -> int {
-            MITOS_TRY((zr2c_pass_tuned<T, NN>(sched.v[TUNE_Z_R2C], ld, K, hs, 1, 0, OpNone(),
-                                              s)));
+            MITOS_TRY((zr2c_pass_tuned<T, NN>(sched.v[TUNE_Z_R2C], ld, K, hs, 1, 0, OpNone(), s)));
             // out of place (an in-place strided pass streams slower)
-            MITOS_TRY((strided_pass_tuned<T, NN, 1, -1>(sched.v[TUNE_Y_FWD], K, a(0), hs, 1,
-                                                        0, OpNone(), s)));
-            return strided_pass_tuned<T, NN, 0, -1>(sched.v[TUNE_X_FWD], a(0), K, hs, 1, 0,
-                                                    OpNone(), s);
+            MITOS_TRY((strided_pass_tuned<T, NN, 1, -1>(sched.v[TUNE_Y_FWD], K, a(0), hs, OpNone(),
+                                                        s)));
+            return strided_pass_tuned<T, NN, 0, -1>(sched.v[TUNE_X_FWD], a(0), K, hs, OpNone(), s);
         };
         auto c2r = [&]() -> int {
-            MITOS_TRY((strided_pass_tuned<T, NN, 0, 1>(sched.v[TUNE_X_FWD], K, a(0), hs, 1, 0,
-                                                       OpNone(), s)));
-            MITOS_TRY((strided_pass_tuned<T, NN, 1, 1>(sched.v[TUNE_Y_FWD], a(0), a(1), hs, 1,
-                                                       0, OpNone(), s)));
+            MITOS_TRY((strided_pass_tuned<T, NN, 0, 1>(sched.v[TUNE_X_FWD], K, a(0), hs, OpNone(), s)));
+            MITOS_TRY((strided_pass_tuned<T, NN, 1, 1>(sched.v[TUNE_Y_FWD], a(0), a(1), hs, OpNone(),
+                                                       s)));
             return zc2r_pass_tuned<T, NN, 0>(sched.v[TUNE_Z_C2R], a(1), real, hs, rs, 1, 0, 0,
                                              (T)1, OpNone(), s);
         };
@@ -300,13 +295,12 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
             }));
             MITOS_TRY(timed(s, "delta2_z_r2c", Rg + G, [&] {
                 RealRowLoader<T> ld{d2, rs2, 0};
-                return zr2c_pass_tuned<T, NN>(sched.v[TUNE_Z_R2C], ld, D, hs, 1, 0, OpNone(),
-                                              s);
+                return zr2c_pass_tuned<T, NN>(sched.v[TUNE_Z_R2C], ld, D, hs, 1, 0, OpNone(), s);
             }));
             // 5. y pass forward of delta2, out of place into a(2)
             MITOS_TRY(timed(s, "delta2_y_fwd", 2 * G, [&] {
-                return strided_pass_tuned<T, NN, 1, -1>(sched.v[TUNE_Y_FWD], D, a(2), hs, 1,
-                                                        0, OpNone(), s);
+                return strided_pass_tuned<T, NN, 1, -1>(sched.v[TUNE_Y_FWD], D, a(2), hs,
+                                                        OpNone(), s);
             }));
             D = a(2);
         } else {
@@ -523,12 +517,10 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
         // y and x out of place through a(0) (free once the displacement
         // grids are made)
         MITOS_TRY(timed(s, "density_y_fwd", 2 * G, [&] {
-            return strided_pass_tuned<T, NN, 1, -1>(sched.v[TUNE_Y_FWD], K, a(0), hs, 1, 0,
-                                                    OpNone(), s);
+            return strided_pass_tuned<T, NN, 1, -1>(sched.v[TUNE_Y_FWD], K, a(0), hs, OpNone(), s);
         }));
         MITOS_TRY(timed(s, "density_x_fwd", 2 * G, [&] {
-            return strided_pass_tuned<T, NN, 0, -1>(sched.v[TUNE_X_FWD], a(0), K, hs, 1, 0,
-                                                    OpNone(), s);
+            return strided_pass_tuned<T, NN, 0, -1>(sched.v[TUNE_X_FWD], a(0), K, hs, OpNone(), s);
         }));
         const double* w2 = window_table(NN, L, 2);
         if (!w2) return MITOS_ERR_ALLOC;

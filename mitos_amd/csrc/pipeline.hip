@@ -293,15 +293,13 @@ template <typename T>
 static int unstencil_psi(Pipe<T>* P, int N, T* out, hipStream_t s) {
     const double* S = smooth_table<double>(N);
     if (!S) return MITOS_ERR_ALLOC;
-    const GridLayout gin{N, P->hs, P->prs()};
-    const GridLayout gout{N, P->hs, (long)N};
     const double norm = 1.0 / ((double)N * N * N);
     const int masks[3] = {7, 6, 4};
     for (int i = 0; i < 3; i++) {
-        RealRowLoader<T> ld{P->psi(i) + MITOS_PSI_SO, gin.rs, 0};
-        MITOS_TRY((r2c_3d<T>(ld, P->K, gin, 1, 0, OpNone(), OpNone(), OpNone(), s)));
-        MITOS_TRY((c2r_3d<T>(P->K, P->a(0), out + (size_t)i * N * N * N, gout, 1, 0, 0, (T)1,
-                             OpUnstencil{S, masks[i], norm}, OpNone(), OpNone(), s)));
+        RealRowLoader<T> ld{P->psi(i) + MITOS_PSI_SO, P->prs(), 0};
+        MITOS_TRY((r2c_3d<T>(N, ld, P->a(0), P->a(1), P->K, P->hs, OpNone(), s)));
+        MITOS_TRY((c2r_3d<T>(N, P->K, P->hs, P->a(0), P->a(1), out + (size_t)i * N * N * N,
+                             (long)N, (T)1, OpUnstencil{S, masks[i], norm}, s)));
     }
     return MITOS_OK;
 }
