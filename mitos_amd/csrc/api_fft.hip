@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/mitos_hip.h"
+#include "dropin.h"
 #include "kspace.h"
 
 using namespace mitos;
@@ -95,7 +96,7 @@ int launch_apply(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double box
     const long n = nx * N * (N / 2 + 1);
     if (n <= 0) return api_sync();
     hipLaunchKernelGGL((k_apply_kernel<TW, TR, HOW>), dim3(nblk(n, kApplyBlock)), dim3(256), 0,
-                       api_stream(), w, r, N, x0, nx, boxlen, ks, tab, t);
+                       api_stream(), w, (long)(N / 2 + 1), r, N, x0, nx, boxlen, ks, tab, t);
     MITOS_TRY(launch_status());
     return api_sync();
 }
@@ -283,70 +284,6 @@ int c2r_plain(int N, const cx<T>* in, T* out, long rs, double scale) {
     return api_sync();
 }
 
-// 2lpt.c:100-116: second-order source from the six Hessian grids (padding included)
-__global__ void k_delta2(double* out, const double* const* h, long n) {
-#pragma clang fp contract(off)
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const double d_dxx = h[0][k], d_dxy = h[1][k], d_dxz = h[2][k];
-    const double d_dyy = h[3][k], d_dyz = h[4][k], d_dzz = h[5][k];
-    out[k] = d_dzz * d_dyy + d_dzz * d_dxx + d_dyy * d_dxx - d_dxy * d_dxy - d_dyz * d_dyz -
-             d_dxz * d_dxz;
-}
-
-// src/monge_ampere.c:124-151: residual (1 + rho) - det(I + Hessian) of every
-// entry (padding included), and per-block sums of resid^2 and rho^2 (tree in
-// a fixed order, so the diagnostic does not depend on scheduling)
-__global__ void __launch_bounds__(256) k_ma_residual(double* out, const double* const* h,
-                                                     const double* rho, long n, double* part) {
-#pragma clang fp contract(off)
-    __shared__ double se[256], sn[256];
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    double e = 0, q = 0;
-    if (k < n) {
-        const double d_dxx = h[0][k], d_dxy = h[1][k], d_dxz = h[2][k];
-        const double d_dyy = h[3][k], d_dyz = h[4][k], d_dzz = h[5][k];
-        const double M0 = 1 + d_dxx, M1 = d_dxy, M2 = d_dxz;
-        const double M3 = d_dxy, M4 = 1 + d_dyy, M5 = d_dyz;
-        const double M6 = d_dxz, M7 = d_dyz, M8 = 1 + d_dzz;
-        // det3 of src/monge_ampere.c:38-42
-        const double det = M0 * (M4 * M8 - M5 * M7) - M1 * (M3 * M8 - M5 * M6) +
-                           M2 * (M3 * M7 - M4 * M6);
-        const double r = rho[k];
-        const double resid = (1 + r) - det;
-        out[k] = resid;
-        e = resid * resid;
-        q = r * r;
-    }
-    se[threadIdx.x] = e;
-    sn[threadIdx.x] = q;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            se[threadIdx.x] += se[threadIdx.x + w];
-            sn[threadIdx.x] += sn[threadIdx.x + w];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = se[0];
-        part[2 * blockIdx.x + 1] = sn[0];
-    }
-}
-
-__global__ void k_add_inplace(double* a, const double* b, long n) {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) a[k] += b[k];
-}
-
-// 2lpt.c:131-133
-__global__ void k_combine(double* pot, const double* work, long n, double f1, double f2) {
-#pragma clang fp contract(off)
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    pot[k] = pot[k] * f1 + f2 * work[k];
-}
-
 }  // namespace
 
 // ---- kernel callbacks (host evaluation; addresses select device kernels) ----------
@@ -436,26 +373,13 @@ extern "C" void kernel_gaussian_inv(struct kernel* the_kernel) {
 
 // ---- FFTs on distributed grids (src/fft.c:219-254) ---------------------------------
 extern "C" int fft_r2c_dg(struct distributed_grid* dg) {
-    if (!dg || !dg->box || !dg->fbox) return set_last_error(MITOS_ERR_ARG);
-    const int N = dg->N;
-    if (!size_supported(N)) return set_last_error(MITOS_ERR_UNSUPPORTED);
-    const double boxvol = dg->boxlen * dg->boxlen * dg->boxlen;
-    const double s = boxvol / ((long long)N * N * N);
-    MITOS_TRY(set_last_error(r2c_issue<double>(N, dg->box, N + 2,
-                                               reinterpret_cast<cx<double>*>(dg->fbox),
-                                               OpScale<double>{s})));
-    dg->momentum_space = 1;
+    MITOS_TRY(set_last_error(dg_r2c_issue(dg, false)));
     return set_last_error(api_sync());
 }
 
 extern "C" int fft_c2r_dg(struct distributed_grid* dg) {
-    if (!dg || !dg->box || !dg->fbox) return set_last_error(MITOS_ERR_ARG);
-    const int N = dg->N;
-    const double boxvol = dg->boxlen * dg->boxlen * dg->boxlen;
-    MITOS_TRY(set_last_error(c2r_plain<double>(
-        N, reinterpret_cast<const cx<double>*>(dg->fbox), dg->box, N + 2, 1.0 / boxvol)));
-    dg->momentum_space = 0;
-    return MITOS_OK;
+    MITOS_TRY(set_last_error(dg_c2r_issue(dg)));
+    return set_last_error(api_sync());
 }
 
 extern "C" int fft_apply_kernel_dg(struct distributed_grid* dg_write,
@@ -567,192 +491,60 @@ extern "C" int mitos_fft_c2r_float(int N, const fftwf_complex* in, float* out) {
 }
 
 // ---- Poisson (src/poisson.c:29-70) --------------------------------------------------------
+namespace mitos {
+
+// r2c with its normalisation and, when asked, the Poisson kernel on the stored
+// modes (include/fft_kernels.h:96-99)
+int dg_r2c_issue(struct distributed_grid* dg, bool poisson) {
+    if (!dg || !dg->box || !dg->fbox) return MITOS_ERR_ARG;
+    const int N = dg->N;
+    const double s = dg->boxlen * dg->boxlen * dg->boxlen / ((long long)N * N * N);
+    cx<double>* out = reinterpret_cast<cx<double>*>(dg->fbox);
+    if (poisson)
+        MITOS_TRY((r2c_issue<double>(N, dg->box, N + 2, out,
+                                     OpScalePoisson{N, s, 2 * M_PI / dg->boxlen})));
+    else
+        MITOS_TRY((r2c_issue<double>(N, dg->box, N + 2, out, OpScale<double>{s})));
+    dg->momentum_space = 1;
+    return MITOS_OK;
+}
+
+int dg_c2r_issue(struct distributed_grid* dg) {
+    if (!dg || !dg->box || !dg->fbox) return MITOS_ERR_ARG;
+    const double boxvol = dg->boxlen * dg->boxlen * dg->boxlen;
+    MITOS_TRY(c2r_issue<double>(dg->N, reinterpret_cast<const cx<double>*>(dg->fbox), dg->box,
+                                dg->N + 2, 1.0 / boxvol));
+    dg->momentum_space = 0;
+    return MITOS_OK;
+}
+
+int apply_padded_issue(cx<double>* w, long whs, const struct distributed_grid* dg,
+                       const KSpec& ks) {
+    const int N = dg->N;
+    const long n = (long)N * N * (N / 2 + 1);
+    hipLaunchKernelGGL((k_apply_kernel<double, double, APPLY_DIRECT>), dim3(nblk(n, kApplyBlock)),
+                       dim3(256), 0, api_stream(), w, whs,
+                       reinterpret_cast<const cx<double>*>(dg->fbox), N, 0L, (long)N, dg->boxlen,
+                       ks, (const double*)nullptr, TransferTab{});
+    return launch_status();
+}
+
+}  // namespace mitos
+
 extern "C" int solvePoisson_dg(struct distributed_grid* dg) {
-    MITOS_TRY(fft_r2c_dg(dg));
-    MITOS_TRY(fft_apply_kernel_dg(dg, dg, kernel_inv_poisson, NULL));
-    return fft_c2r_dg(dg);
+    MITOS_TRY(set_last_error(dg_r2c_issue(dg, true)));
+    MITOS_TRY(set_last_error(dg_c2r_issue(dg)));
+    return set_last_error(api_sync());
 }
 
 extern "C" int solvePoisson(double* phi, double* f, int N, double boxlen) {
     if (!phi || !f) return set_last_error(MITOS_ERR_ARG);
     cx<double>* fbox = (cx<double>*)workspace(1, sizeof(cx<double>) * half_elems(N));
     if (!fbox) return set_last_error(MITOS_ERR_ALLOC);
-    fftw_complex* fb = reinterpret_cast<fftw_complex*>(fbox);
-    MITOS_TRY(mitos_fft_r2c(N, f, fb));
-    MITOS_TRY(fft_normalize_r2c(fb, N, boxlen));
-    MITOS_TRY(fft_apply_kernel(fb, fb, N, boxlen, kernel_inv_poisson, NULL));
-    MITOS_TRY(mitos_fft_c2r(N, fb, phi));
-    return fft_normalize_c2r(phi, N, boxlen);
-}
-
-// ---- 2LPT (src/2lpt.c:38-143) --------------------------------------------------------------
-extern "C" int solve2LPT(struct distributed_grid* potential, struct distributed_grid* density,
-                         struct distributed_grid* workspace_grid, double factor1,
-                         double factor2) {
-    if (!potential || !density || !workspace_grid) return set_last_error(MITOS_ERR_ARG);
-    const int N = density->N;
-    // src/2lpt.c:54-60 (asserts in the reference)
-    if (potential->NX != density->NX || density->NX != workspace_grid->NX ||
-        potential->X0 != density->X0 || density->X0 != workspace_grid->X0 ||
-        potential->N != density->N || density->N != workspace_grid->N)
-        return set_last_error(MITOS_ERR_DIMS);
-    if (potential->box == density->box || workspace_grid->box == density->box ||
-        potential->box == workspace_grid->box)
-        return set_last_error(MITOS_ERR_ARG);
-    // src/2lpt.c:69-72 returns 1 here (fft_apply_kernel_dg returns 2 for the
-    // same condition, src/fft.c:274)
-    if (density->momentum_space != 1) return set_last_error(1);
-
-    void (*const derivatives[3])(struct kernel*) = {kernel_dx, kernel_dy, kernel_dz};
-    const int index_a[] = {0, 0, 0, 1, 1, 2};
-    const int index_b[] = {0, 1, 2, 1, 2, 2};
-
-    MITOS_TRY(fft_apply_kernel_dg(potential, density, kernel_inv_poisson, NULL));
-    MITOS_TRY(fft_r2c_dg(density));  // src/2lpt.c:78
-
-    const long padded = (long)N * N * (N + 2);
-    double* hess[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    struct distributed_grid d;
-    memset(&d, 0, sizeof(d));
-    int rc = MITOS_OK;
-    for (int j = 0; j < 6 && rc == MITOS_OK; j++)
-        if (!(hess[j] = (double*)pool_alloc(sizeof(double) * padded))) rc = MITOS_ERR_ALLOC;
-    if (rc == MITOS_OK) rc = alloc_local_grid(&d, N, density->boxlen, density->comm);
-    double** hdev = nullptr;
-    if (rc == MITOS_OK && hipMalloc(&hdev, sizeof(double*) * 6) != hipSuccess)
-        rc = MITOS_ERR_ALLOC;
-    for (int j = 0; j < 6 && rc == MITOS_OK; j++) {
-        rc = fft_apply_kernel_dg(&d, potential, derivatives[index_a[j]], NULL);
-        if (rc == MITOS_OK) rc = fft_apply_kernel_dg(&d, &d, derivatives[index_b[j]], NULL);
-        if (rc == MITOS_OK) rc = fft_c2r_dg(&d);
-        // on the library stream: the next derivative overwrites d
-        if (rc == MITOS_OK &&
-            hipMemcpyAsync(hess[j], d.box, sizeof(double) * padded, hipMemcpyDeviceToDevice,
-                           api_stream()) != hipSuccess)
-            rc = MITOS_ERR_DEVICE;
-    }
-    if (rc == MITOS_OK &&
-        copy_sync(hdev, hess, sizeof(double*) * 6, hipMemcpyHostToDevice) != hipSuccess)
-        rc = MITOS_ERR_DEVICE;
-    if (rc == MITOS_OK) {
-        hipLaunchKernelGGL(k_delta2, dim3(nblk(padded)), dim3(256), 0, api_stream(),
-                           workspace_grid->box, (const double* const*)hdev, padded);
-        rc = launch_status();
-        if (rc == MITOS_OK) rc = api_sync();
-    }
-    free_local_grid(&d);
-    if (hdev) hipFree(hdev);
-    for (int j = 0; j < 6; j++)
-        pool_free(hess[j]);
-    if (rc != MITOS_OK) return set_last_error(rc);
-
-    MITOS_TRY(solvePoisson_dg(workspace_grid));
-    MITOS_TRY(fft_c2r_dg(potential));
-    hipLaunchKernelGGL(k_combine, dim3(nblk(padded)), dim3(256), 0, api_stream(), potential->box,
-                       workspace_grid->box, padded, factor1, factor2);
-    MITOS_TRY(set_last_error(launch_status()));
-    MITOS_TRY(set_last_error(api_sync()));
-    return fft_r2c_dg(potential);
-}
-
-// ---- Monge-Ampere (src/monge_ampere.c:50-183) -----------------------------------------------
-namespace {
-thread_local std::vector<double> g_ma_eps;
-}
-
-extern "C" int solveMongeAmpere(struct distributed_grid* potential,
-                                struct distributed_grid* density,
-                                struct distributed_grid* workspace_grid, int cycles) {
-    if (!potential || !density || !workspace_grid || cycles < 0)
-        return set_last_error(MITOS_ERR_ARG);
-    const int N = density->N;
-    // src/monge_ampere.c:68-74 (asserts in the reference)
-    if (potential->NX != density->NX || density->NX != workspace_grid->NX ||
-        potential->X0 != density->X0 || density->X0 != workspace_grid->X0 ||
-        potential->N != density->N || density->N != workspace_grid->N)
-        return set_last_error(MITOS_ERR_DIMS);
-    if (potential->box == density->box || workspace_grid->box == density->box ||
-        potential->box == workspace_grid->box)
-        return set_last_error(MITOS_ERR_ARG);
-    if (density->momentum_space != 1) return set_last_error(1);  // :82-85
-    g_ma_eps.clear();
-
-    void (*const derivatives[3])(struct kernel*) = {kernel_dx, kernel_dy, kernel_dz};
-    const int index_a[] = {0, 0, 0, 1, 1, 2};
-    const int index_b[] = {0, 1, 2, 1, 2, 2};
-    MITOS_TRY(fft_apply_kernel_dg(potential, density, kernel_inv_poisson, NULL));
-    MITOS_TRY(fft_r2c_dg(density));  // :91 (as src/2lpt.c:78)
-    if (cycles == 0) return MITOS_OK;
-
-    const long padded = (long)N * N * (N + 2);
-    const unsigned nb = nblk(padded);
-    double* hess[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    double** hdev = nullptr;
-    double* part = nullptr;
-    struct distributed_grid d;
-    memset(&d, 0, sizeof(d));
-    int rc = MITOS_OK;
-    for (int j = 0; j < 6 && rc == MITOS_OK; j++)
-        if (!(hess[j] = (double*)pool_alloc(sizeof(double) * padded))) rc = MITOS_ERR_ALLOC;
-    if (rc == MITOS_OK && (hipMalloc(&hdev, sizeof(double*) * 6) != hipSuccess ||
-                           hipMalloc(&part, sizeof(double) * 2 * nb) != hipSuccess))
-        rc = MITOS_ERR_ALLOC;
-    if (rc == MITOS_OK) rc = alloc_local_grid(&d, N, density->boxlen, density->comm);
-    if (rc == MITOS_OK &&
-        copy_sync(hdev, hess, sizeof(double*) * 6, hipMemcpyHostToDevice) != hipSuccess)
-        rc = MITOS_ERR_DEVICE;
-    std::vector<double> hp(2 * (size_t)nb);
-    for (int it = 0; it < cycles && rc == MITOS_OK; it++) {
-        // the six Hessian components (:103-117)
-        for (int j = 0; j < 6 && rc == MITOS_OK; j++) {
-            rc = fft_apply_kernel_dg(&d, potential, derivatives[index_a[j]], NULL);
-            if (rc == MITOS_OK) rc = fft_apply_kernel_dg(&d, &d, derivatives[index_b[j]], NULL);
-            if (rc == MITOS_OK) rc = fft_c2r_dg(&d);
-            if (rc == MITOS_OK &&
-                hipMemcpyAsync(hess[j], d.box, sizeof(double) * padded, hipMemcpyDeviceToDevice,
-                               api_stream()) != hipSuccess)
-                rc = MITOS_ERR_DEVICE;
-        }
-        if (rc != MITOS_OK) break;
-        // residuals (:120-151)
-        hipLaunchKernelGGL(k_ma_residual, dim3(nb), dim3(256), 0, api_stream(),
-                           workspace_grid->box, (const double* const*)hdev, density->box, padded,
-                           part);
-        rc = launch_status();
-        if (rc == MITOS_OK &&
-            (hipMemcpyAsync(hp.data(), part, sizeof(double) * 2 * nb, hipMemcpyDeviceToHost,
-                            api_stream()) != hipSuccess ||
-             hipStreamSynchronize(api_stream()) != hipSuccess))
-            rc = MITOS_ERR_DEVICE;
-        if (rc != MITOS_OK) break;
-        double eps = 0, norm = 0;
-        for (unsigned b = 0; b < nb; b++) {
-            eps += hp[2 * b];
-            norm += hp[2 * b + 1];
-        }
-        // (:159-172) Poisson solve of the residual, added to the potential
-        rc = solvePoisson_dg(workspace_grid);
-        if (rc == MITOS_OK) rc = fft_c2r_dg(potential);
-        if (rc == MITOS_OK) {
-            hipLaunchKernelGGL(k_add_inplace, dim3(nb), dim3(256), 0, api_stream(),
-                               potential->box, workspace_grid->box, padded);
-            rc = launch_status();
-        }
-        if (rc == MITOS_OK) rc = api_sync();
-        if (rc == MITOS_OK) rc = fft_r2c_dg(potential);
-        // (:183-186) root-mean-square residual relative to the source
-        g_ma_eps.push_back(sqrt((eps / norm) / ((double)N * N * N)));
-    }
-    free_local_grid(&d);
-    if (hdev) hipFree(hdev);
-    if (part) hipFree(part);
-    for (int j = 0; j < 6; j++)
-        pool_free(hess[j]);
-    return set_last_error(rc);
-}
-
-extern "C" int mitos_monge_ampere_residuals(double* rms_eps, int n) {
-    const int m = (int)g_ma_eps.size();
-    for (int i = 0; i < n && i < m && rms_eps; i++) rms_eps[i] = g_ma_eps[i];
-    return m;
+    const double boxvol = boxlen * boxlen * boxlen;
+    const double s = boxvol / ((long long)N * N * N);
+    MITOS_TRY(set_last_error(
+        (r2c_issue<double>(N, f, N, fbox, OpScalePoisson{N, s, 2 * M_PI / boxlen}))));
+    MITOS_TRY(set_last_error((c2r_issue<double>(N, fbox, phi, N, 1.0 / boxvol))));
+    return set_last_error(api_sync());
 }

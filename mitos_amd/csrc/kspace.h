@@ -184,11 +184,11 @@ __device__ __forceinline__ void for_block_modes(int N, long x0, long nx, LOAD&& 
 enum { APPLY_DIRECT = 0, APPLY_WINDOW = 1, APPLY_RADIAL = 2, APPLY_TRANSFER = 3 };
 
 // TW/TR may be float (the _float variants compute the product in double, as C
-// does for fftwf_complex * double complex).
+// does for fftwf_complex * double complex).  r is dense, w has rows of whs.
 template <typename TW, typename TR, int HOW>
 __global__ void __launch_bounds__(256)
-    k_apply_kernel(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double boxlen, KSpec ks,
-                   const double* __restrict__ tab, TransferTab t) {
+    k_apply_kernel(cx<TW>* w, long whs, const cx<TR>* r, int N, long x0, long nx, double boxlen,
+                   KSpec ks, const double* __restrict__ tab, TransferTab t) {
 #pragma clang fp contract(off)
     const double dk = 2 * M_PI / boxlen;
     auto load = [&](long id) { return ld(r + id); };
@@ -213,7 +213,8 @@ __global__ void __launch_bounds__(256)
             kv = mk<double>(tab[(long)nx_ * nx_ + (long)ny * ny + (long)z * z], 0);
         }
         const double re = (double)a.re, im = (double)a.im;
-        st(w + id, mk<TW>((TW)(re * kv.re - im * kv.im), (TW)(re * kv.im + im * kv.re)));
+        st(w + (((long)x - x0) * N + y) * whs + z,
+           mk<TW>((TW)(re * kv.re - im * kv.im), (TW)(re * kv.im + im * kv.re)));
     });
 }
 
@@ -235,6 +236,18 @@ static __global__ void k_radial_values(KSpec ks, long n, double boxlen, double* 
     const double dk = 2 * M_PI / boxlen;
     tab[i] = ksp_value(ks, 0, 0, 0, sqrt((double)i) * dk).re;
 }
+
+// r2c operator: normalisation, then the Poisson kernel -1/k^2 (1 at k = 0)
+struct OpScalePoisson {
+    int N;
+    double s, dk;
+    __device__ __forceinline__ cx<double> pre(cx<double> v, int, int, int) const { return v; }
+    __device__ __forceinline__ cx<double> post(cx<double> v, int x, int y, int z) const {
+        const double kx = freq_index(x, N) * dk, ky = freq_index(y, N) * dk, kz = z * dk;
+        const double k2 = kx * kx + ky * ky + kz * kz;
+        return cscale(v, k2 > 0 ? -s / k2 : s);
+    }
+};
 
 // write = read * m over nx x-slabs, m the kernel values evaluated on the host
 // (dense N x N x (N/2+1) per slab)

@@ -2,73 +2,10 @@
 // once per precision by pipe_f32.hip and pipe_f64.hip.
 #pragma once
 
+#include "multi_launch.h"
 #include "pipe.h"
 
 namespace mitos {
-
-// ---- launch helpers for the fused kernels ---------------------------------------------
-// Line configuration and tile width of the register-heavy multi-transform
-// kernels: 8 (or 12) values per thread and 64-byte tile rows, so that the
-// input tile, the transformed copy and the radix temporaries stay in VGPRs.
-// Multi-output passes on float lines of 1024: 16 values per thread, so a
-// line is one wave (fewer exchange steps), and 128-byte tile rows (whole
-// lines; work-groups of 1024 threads, one per CU); the combine pass keeps the
-// smaller line configuration (MULTI = false).
-template <typename T, int L, bool MULTI = true>
-struct HeavyCfg {
-    static constexpr bool WIDE = MULTI && sizeof(T) == 4 && L == 1024;
-    typedef typename std::conditional<WIDE, LineCfg<L>, LineCfgS<L>>::type CFG;
-    static constexpr int E = CFG::E;
-    static constexpr int TPL = L / E;
-    static constexpr int C0 = (WIDE ? 128 : 64) / (2 * (int)sizeof(T));
-    static constexpr int C = (TPL * C0 <= 1024) ? C0 : 1024 / TPL;
-};
-template <typename T, int L, int AXIS, int DIR, int NIN, typename CODES,
-          typename RAD = typename HeavyCfg<T, L>::CFG::R>
-struct MultiK;
-template <typename T, int L, int AXIS, int DIR, int NIN, typename CODES, int... Rs>
-struct MultiK<T, L, AXIS, DIR, NIN, CODES, Radices<Rs...>> {
-    static int go(const MultiPtrs<T, NIN, CODES::n>& P, long hs, double dk, hipStream_t s) {
-        constexpr int C = HeavyCfg<T, L>::C;
-        constexpr int E = HeavyCfg<T, L>::E;
-        // one exchange buffer per component unless that leaves less than two
-        // work-groups per CU; the wide form runs one per CU by its registers
-        // anyway (1024 threads at about 124), so it takes both (139 KB)
-        constexpr bool SPLIT = !HeavyCfg<T, L>::WIDE &&
-                               2 * LdsMap<T, L, C, true>::SIZE * sizeof(T) > 81920;
-        const int ncols = L / 2 + 1;
-        const cx<T>* tw = twiddles<T>(L);
-        if (!tw) return MITOS_ERR_ALLOC;
-        constexpr int KO = (AXIS == 0 && L >= 64) ? 2 : 1;
-        hipLaunchKernelGGL((k_multi_strided<T, L, E, C, AXIS, DIR, SPLIT, NIN, CODES, KO, Rs...>),
-                           dim3((ncols + C - 1) / C, L / KO), dim3(L / E * C), 0, s, P, hs, ncols,
-                           dk, tw);
-        return launch_status();
-    }
-};
-
-template <typename T, int N, typename RAD = typename LineCfgS<N / 2>::R>
-struct HessZK;
-template <typename T, int N, int... Rs>
-struct HessZK<T, N, Radices<Rs...>> {
-    // delta2 rows written as reals (row stride rs) for a separate z pass
-    static int go(const MultiPtrs<T, 6, 1>& P, long hs, double dk, T scale, T* real, long rs,
-                  hipStream_t s) {
-        constexpr int L = N / 2;
-        constexpr int E = LineCfgS<L>::E;
-        constexpr int TPL = L / E;
-        // a row of a wave or more: one row per work-group (no barrier waits
-        // on other rows' waves)
-        constexpr int RW = TPL >= 64 ? 1 : RowsPerBlock<TPL>::value;
-        const long nrows = (long)N * N;
-        const cx<T>* tw = twiddles<T>(L);
-        const cx<T>* twN = twiddles<T>(N);
-        if (!tw || !twN) return MITOS_ERR_ALLOC;
-        hipLaunchKernelGGL((k_hess_z<T, L, E, RW, Rs...>), dim3(nblk(nrows, RW)),
-                           dim3(TPL * RW), 0, s, P, nrows, hs, dk, scale, tw, twN, real, rs);
-        return launch_status();
-    }
-};
 
 template <typename T, int N, typename RAD = typename HeavyCfg<T, N, false>::CFG::R>
 struct CombineK;
