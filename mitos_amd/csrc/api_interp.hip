@@ -63,38 +63,6 @@ __global__ void k_grid_tsc_slices(Slices s, double x, double y, double z, double
     *out = sum;
 }
 
-// src/mitos.c:827-863 (three sequential moves), :867-907 (velocities by TSC
-// at the moved, not yet wrapped positions, stored as float), :1072-1077 (wrap)
-__global__ void __launch_bounds__(256)
-    k_displace_velocity(const double* __restrict__ px, const double* __restrict__ py,
-                        const double* __restrict__ pz, const double* __restrict__ vx,
-                        const double* __restrict__ vy, const double* __restrict__ vz, int N,
-                        double boxlen, long long npart, float* X, float* Y, float* Z,
-                        float* VX, float* VY, float* VZ) {
-#pragma clang fp contract(off)
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npart) return;
-    const unsigned rs = (unsigned)(N + 2);
-    const float invN = 1.0f / N;
-    float x = X[p], y = Y[p], z = Z[p];
-    if (px) {
-        double d = tsc_gather<double, double, false>(px, rs, N, invN, boxlen, x, y, z);
-        x = (float)((double)x - d);
-        d = tsc_gather<double, double, false>(py, rs, N, invN, boxlen, x, y, z);
-        y = (float)((double)y - d);
-        d = tsc_gather<double, double, false>(pz, rs, N, invN, boxlen, x, y, z);
-        z = (float)((double)z - d);
-    }
-    if (vx) {
-        VX[p] = (float)tsc_gather<double, double, false>(vx, rs, N, invN, boxlen, x, y, z);
-        VY[p] = (float)tsc_gather<double, double, false>(vy, rs, N, invN, boxlen, x, y, z);
-        VZ[p] = (float)tsc_gather<double, double, false>(vz, rs, N, invN, boxlen, x, y, z);
-    }
-    X[p] = (float)fwrap_fast(x, boxlen);
-    Y[p] = (float)fwrap_fast(y, boxlen);
-    Z[p] = (float)fwrap_fast(z, boxlen);
-}
-
 // the export arrays of src/mitos.c:1097-1107 for particles [p0, p0+n)
 __global__ void k_pack(long long n, long long p0, const float* X, const float* Y, const float* Z,
                        const float* VX, const float* VY, const float* VZ, double mass,
@@ -190,11 +158,15 @@ extern "C" int mitos_displace_velocity_tsc_dg(
     if (npart == 0) return MITOS_OK;
     if ((unsigned long long)(N + 2) * N * N > 0xffffffffULL)
         return set_last_error(MITOS_ERR_UNSUPPORTED);
-    hipLaunchKernelGGL(k_displace_velocity, dim3(nblk(npart)), dim3(256), 0, api_stream(),
-                       disp ? psi_x->box : nullptr, disp ? psi_y->box : nullptr,
-                       disp ? psi_z->box : nullptr, vel ? vel_x->box : nullptr,
-                       vel ? vel_y->box : nullptr, vel ? vel_z->box : nullptr, N, g0->boxlen,
-                       npart, X, Y, Z, VX, VY, VZ);
+    DisplaceGrids g{};
+    for (int i = 0; i < 3; i++) {
+        if (disp) g.psi[i] = all[i]->box;
+        if (vel) g.vel[i] = all[3 + i]->box;
+    }
+    auto launch = disp && vel ? displace_grids_launch<true, true>
+                  : disp      ? displace_grids_launch<true, false>
+                              : displace_grids_launch<false, true>;
+    launch(g, N, g0->boxlen, npart, X, Y, Z, VX, VY, VZ, api_stream());
     MITOS_TRY(set_last_error(launch_status()));
     return set_last_error(api_sync());
 }

@@ -256,9 +256,9 @@ extern "C" int mitos_displace_tsc_dg(const struct distributed_grid* psi_x,
     // the gather indexes a grid with 32-bit element offsets
     if ((unsigned long long)(N + 2) * N * N > 0xffffffffULL)
         return set_last_error(MITOS_ERR_UNSUPPORTED);
-    hipLaunchKernelGGL((k_displace<double>), dim3(nblk(npart)), dim3(256), 0, api_stream(),
-                       psi_x->box, psi_y->box, psi_z->box, (unsigned)(N + 2), N, psi_x->boxlen,
-                       npart, X, Y, Z);
+    const DisplaceGrids g{{psi_x->box, psi_y->box, psi_z->box}, {}};
+    displace_grids_launch<true, false>(g, N, psi_x->boxlen, npart, X, Y, Z, nullptr, nullptr,
+                                       nullptr, api_stream());
     MITOS_TRY(set_last_error(launch_status()));
     return set_last_error(api_sync());
 }

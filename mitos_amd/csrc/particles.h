@@ -63,6 +63,28 @@ __device__ __forceinline__ void tsc_axis(M X, int& i0, M w[3]) {
     }
 }
 
+// tsc_axis in half the instructions, the same bits.  The reference forms xx =
+// |X - tap| and picks its formula by xx < 1/2 and xx < 3/2.  With u = X - (nearest
+// tap), exact in floating point, the taps lie at 1 + u, |u| and 1 - u (the
+// reference's xx, each rounded once as there), and the formulas are known: where
+// two meet, at xx = 1/2, they agree.  A cell past the int range, an infinity or a
+// NaN has all weights zero, as there.  For the kernels that read their taps from
+// memory; k_displace_tile_ref, held to 128 registers, is slower with it (512^3:
+// 24.3 -> 25.3 ms for the realization).
+__device__ __forceinline__ void tsc_axis_short(double X, int& i0, double w[3]) {
+#pragma clang fp contract(off)
+    const int iX = (int)floor(X);
+    const double d = X - iX;
+    const bool low = d < 0.5;  // reference loops from floor(d-1.5)
+    i0 = low ? iX - 1 : iX;
+    const double u = low ? d : d - 1;
+    const bool ok = fabs(u) <= 0.5;
+    const double l = 1.5 - (1 + u), r = 1.5 - (1 - u);
+    w[0] = ok ? 0.5 * l * l : 0;
+    w[1] = ok ? 0.75 - u * u : 0;
+    w[2] = ok ? 0.5 * r * r : 0;
+}
+
 __device__ __forceinline__ int wrapi(int i, int N) { return ((i % N) + N) % N; }
 // wrap of an index known to lie in [-N, 2N)
 __device__ __forceinline__ int wrap1(int i, int N) { return i < 0 ? i + N : (i >= N ? i - N : i); }
@@ -76,49 +98,75 @@ __device__ __forceinline__ int wrapf(int i, int N, float invN) {
 }
 
 // gridTSC_dg (src/grids_interp.c:267-309) on one rank: all taps wrap
-// periodically.  The 27 taps with nonzero weight are summed in the reference's
-// loop order; FMA = false keeps every product and sum separately rounded (the
-// reference's arithmetic), FMA = true fuses them (FP32 variant).  Element
-// offsets are 32-bit (rs * N * N < 2^32).
-template <typename T, typename M, bool FMA>
-__device__ __forceinline__ M tsc_gather(const T* __restrict__ box, unsigned rs, int N, float invN,
-                                        M boxlen, M x, M y, M z) {
-#pragma clang fp contract(off)
-    const M X = x * N / boxlen;
-    const M Y = y * N / boxlen;
-    const M Z = z * N / boxlen;
-    int i0, j0, k0;
-    M wx[3], wy[3], wz[3];
-    tsc_axis(X, i0, wx);
-    tsc_axis(Y, j0, wy);
-    tsc_axis(Z, k0, wz);
-    const int ib = wrapf(i0, N, invN), jb = wrapf(j0, N, invN), kb = wrapf(k0, N, invN);
-    unsigned ox[3], oy[3], oz[3];
-    const unsigned plane = (unsigned)N * rs;
+// periodically, and the 27 taps with non-zero weight are summed in the
+// reference's loop order with every product and sum separately rounded.
+// One axis of a position: the weights and the taps' byte offsets.  O: unsigned
+// where the grid's bytes fit 32 bits (each load is then the grid's address in
+// scalar registers plus one 32-bit register), else 64-bit.
+template <typename O>
+struct TscTaps {
+    double w[3];
+    O o[3];
+};
+template <typename O>
+__device__ __forceinline__ TscTaps<O> tsc_taps(double X, int N, float invN, O stride) {
+    TscTaps<O> t;
+    int i0;
+    tsc_axis_short(X, i0, t.w);
+    int b = wrapf(i0, N, invN);
+    if ((unsigned)b >= (unsigned)N) b = wrapi(i0, N);  // far outside the box
 #pragma unroll
-    for (int t = 0; t < 3; t++) {
-        ox[t] = (unsigned)wrap1(ib + t, N) * plane;
-        oy[t] = (unsigned)wrap1(jb + t, N) * rs;
-        oz[t] = (unsigned)wrap1(kb + t, N);
-    }
-    M sum = 0;
+    for (int k = 0; k < 3; k++) t.o[k] = (O)wrap1(b + k, N) * stride;
+    return t;
+}
+
+// the sums of G grids at one position.  FLAT: the z taps of all the wave's lanes
+// are consecutive (no lane wraps), so a row is one 16-byte and one 8-byte load;
+// that pays with velocities (250^3 particles on 256^3, moves and velocities: 3.20
+// -> 2.54 ms) and not for moves alone (512^3: 7.76 -> 8.30 ms).
+template <int G, bool FLAT, typename O>
+__device__ __forceinline__ void tsc_sums(const double* const* box, const TscTaps<O>& x,
+                                         const TscTaps<O>& y, const TscTaps<O>& z, double* sum) {
+#pragma clang fp contract(off)
+    typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
+#pragma unroll
+    for (int g = 0; g < G; g++) sum[g] = 0;
 #pragma unroll
     for (int a = 0; a < 3; a++) {
 #pragma unroll
         for (int b = 0; b < 3; b++) {
-            const unsigned row = ox[a] + oy[b];
-            const M wab = wx[a] * wy[b];
+            const O row = x.o[a] + y.o[b];
+            const double wab = x.w[a] * y.w[b];
+            const double w0 = wab * z.w[0], w1 = wab * z.w[1], w2 = wab * z.w[2];
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const M v = (M)box[row + oz[c]];
-                if (FMA)
-                    sum = fma(v, wab * wz[c], sum);
-                else
-                    sum += v * (wab * wz[c]);
+            for (int g = 0; g < G; g++) {
+                const char* p = reinterpret_cast<const char*>(box[g]);
+                double v0, v1, v2;
+                if constexpr (FLAT) {
+                    const pair v = *reinterpret_cast<const pair*>(p + (O)(row + z.o[0]));
+                    v0 = v.x;
+                    v1 = v.y;
+                    v2 = *reinterpret_cast<const double*>(p + (O)(row + z.o[0] + 16));
+                } else {
+                    v0 = *reinterpret_cast<const double*>(p + (O)(row + z.o[0]));
+                    v1 = *reinterpret_cast<const double*>(p + (O)(row + z.o[1]));
+                    v2 = *reinterpret_cast<const double*>(p + (O)(row + z.o[2]));
+                }
+                sum[g] += v0 * w0;
+                sum[g] += v1 * w1;
+                sum[g] += v2 * w2;
             }
         }
     }
-    return sum;
+}
+template <int G, bool FLAT, typename O>
+__device__ __forceinline__ void tsc_gather(const double* const* box, const TscTaps<O>& x,
+                                           const TscTaps<O>& y, const TscTaps<O>& z,
+                                           double* sum) {
+    if (FLAT && __ballot(z.o[2] != z.o[0] + 16) == 0)
+        tsc_sums<G, true>(box, x, y, z, sum);
+    else
+        tsc_sums<G, false>(box, x, y, z, sum);
 }
 
 // src/particle.c:87-129: lattice position of particle p (index x*M*M+y*M+z)
@@ -146,37 +194,107 @@ __global__ void k_lattice(int M, float spacing, long long first_id, float* X, fl
     if (ids) ids[p] = p + first_id;
 }
 
-// one particle: three sequential TSC displacements (src/mitos.c:827-863) then
-// the periodic wrap (:1072-1077), in the reference's double arithmetic
-template <typename T>
-__device__ __forceinline__ void displace_one(const T* __restrict__ px, const T* __restrict__ py,
-                                             const T* __restrict__ pz, unsigned rs, int N,
-                                             double boxlen, float& x, float& y, float& z) {
-#pragma clang fp contract(off)
-    const float invN = 1.0f / N;
-    double d = tsc_gather<T, double, false>(px, rs, N, invN, boxlen, x, y, z);
-    x = (float)((double)x - d);
-    d = tsc_gather<T, double, false>(py, rs, N, invN, boxlen, x, y, z);
-    y = (float)((double)y - d);
-    d = tsc_gather<T, double, false>(pz, rs, N, invN, boxlen, x, y, z);
-    z = (float)((double)z - d);
-    x = (float)fwrap_fast(x, boxlen);
-    y = (float)fwrap_fast(y, boxlen);
-    z = (float)fwrap_fast(z, boxlen);
+// Order in which the particle kernels of the drop-in calls walk their arrays.
+// Particles written by mitos_lattice lie in lattice order, where 256 neighbours
+// in memory are a thin line along z; the taps of a compact block share far more
+// lines.  So an array of M^3 particles is walked in blocks of 8 x 8 x 16 of its
+// lattice indices (any other length in memory order).  This is an order of work
+// only: each particle's result is its own.
+struct ParticleOrder {
+    long long n;
+    int M;  // 0: memory order
+    unsigned nty, ntz, blocks;
+};
+inline ParticleOrder particle_order(long long n) {
+    ParticleOrder o{n, 0, 0, 0, (unsigned)((n + 1023) / 1024)};
+    long long M = (long long)llround(cbrt((double)n));
+    if (M >= 16 && M * M * M == n) {
+        o.M = (int)M;
+        o.nty = (unsigned)((M + 7) / 8);
+        o.ntz = (unsigned)((M + 15) / 16);
+        o.blocks = (unsigned)((M + 7) / 8) * o.nty * o.ntz;
+    }
+    return o;
+}
+// particle k (0..3) of a thread of 256, or -1
+__device__ __forceinline__ long long ordered_particle(const ParticleOrder& o, unsigned block,
+                                                      int k) {
+    if (o.M == 0) {
+        const long long p = (long long)block * 1024 + k * 256 + threadIdx.x;
+        return p < o.n ? p : -1;
+    }
+    const int z = (int)(block % o.ntz) * 16 + (int)(threadIdx.x & 15);
+    const int y = (int)(block / o.ntz % o.nty) * 8 + (int)((threadIdx.x >> 4) & 7);
+    const int x = (int)(block / (o.ntz * o.nty)) * 8 + (int)(threadIdx.x >> 7) + 2 * k;
+    if (x >= o.M || y >= o.M || z >= o.M) return -1;
+    return ((long long)x * o.M + y) * o.M + z;
 }
 
-// particles at X/Y/Z displaced through grids of row stride rs (no halo)
-template <typename T>
-__global__ void __launch_bounds__(256)
-    k_displace(const T* __restrict__ px, const T* __restrict__ py, const T* __restrict__ pz,
-               unsigned rs, int N, double boxlen, long long npart, float* X, float* Y, float* Z) {
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npart) return;
-    float x = X[p], y = Y[p], z = Z[p];
-    displace_one<T>(px, py, pz, rs, N, boxlen, x, y, z);
-    X[p] = x;
-    Y[p] = y;
-    Z[p] = z;
+// The particle loop of src/mitos.c:824-908 and :1072-1077 over padded grids (rows
+// of N + 2): the three sequential moves (DISP), velocities by TSC at the moved,
+// not yet wrapped positions, stored as float (VEL), and the wrap, in the
+// reference's double arithmetic.  A move changes one coordinate, so one axis is
+// formed anew per gather; the three velocities share their taps.  Bound by the L1
+// cache's line accesses (33 per load, 0.83 per cycle and CU: neighbours' taps lie
+// in different rows once they moved) and, at half the time, by the FP64 sums.
+// Against one particle per thread in memory order: 512^3 moves 11.5 -> 7.8 ms,
+// 250^3 moves and velocities on 256^3 4.0 -> 2.5 ms.  Staging the taps' box of
+// 1024 particles in LDS measured 9.4 and 3.6 ms (80 KB windows leave two
+// work-groups per CU to hide the loads of each stage).
+struct DisplaceGrids {
+    const double* psi[3];
+    const double* vel[3];
+};
+template <bool DISP, bool VEL, typename O>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+    k_displace_grids(DisplaceGrids g, int N, double boxlen, ParticleOrder order, float* X,
+                     float* Y, float* Z, float* VX, float* VY, float* VZ) {
+#pragma clang fp contract(off)
+    const unsigned block = xcd_block(blockIdx.x, gridDim.x);
+    const float invN = 1.0f / N;
+    const O sz = 8, sy = (O)(N + 2) * 8, sx = sy * (O)N;
+#pragma unroll 1
+    for (int k = 0; k < 4; k++) {
+        const long long p = ordered_particle(order, block, k);
+        if (p < 0) continue;
+        float x = X[p], y = Y[p], z = Z[p];
+        TscTaps<O> tx = tsc_taps<O>((double)x * N / boxlen, N, invN, sx);
+        TscTaps<O> ty = tsc_taps<O>((double)y * N / boxlen, N, invN, sy);
+        TscTaps<O> tz = tsc_taps<O>((double)z * N / boxlen, N, invN, sz);
+        double d[3];
+        if constexpr (DISP) {
+            tsc_gather<1, VEL>(&g.psi[0], tx, ty, tz, d);
+            x = (float)((double)x - d[0]);
+            tx = tsc_taps<O>((double)x * N / boxlen, N, invN, sx);
+            tsc_gather<1, VEL>(&g.psi[1], tx, ty, tz, d);
+            y = (float)((double)y - d[0]);
+            ty = tsc_taps<O>((double)y * N / boxlen, N, invN, sy);
+            tsc_gather<1, VEL>(&g.psi[2], tx, ty, tz, d);
+            z = (float)((double)z - d[0]);
+        }
+        if constexpr (VEL) {
+            if constexpr (DISP) tz = tsc_taps<O>((double)z * N / boxlen, N, invN, sz);
+            tsc_gather<3, VEL>(g.vel, tx, ty, tz, d);
+            VX[p] = (float)d[0];
+            VY[p] = (float)d[1];
+            VZ[p] = (float)d[2];
+        }
+        X[p] = (float)fwrap_fast(x, boxlen);
+        Y[p] = (float)fwrap_fast(y, boxlen);
+        Z[p] = (float)fwrap_fast(z, boxlen);
+    }
+}
+template <bool DISP, bool VEL>
+inline void displace_grids_launch(const DisplaceGrids& g, int N, double boxlen, long long npart,
+                                  float* X, float* Y, float* Z, float* VX, float* VY, float* VZ,
+                                  hipStream_t s) {
+    const ParticleOrder order = particle_order(npart);
+    if ((unsigned long long)(N + 2) * N * N * 8 < (1ull << 32))
+        hipLaunchKernelGGL((k_displace_grids<DISP, VEL, unsigned>), dim3(order.blocks), dim3(256),
+                           0, s, g, N, boxlen, order, X, Y, Z, VX, VY, VZ);
+    else
+        hipLaunchKernelGGL((k_displace_grids<DISP, VEL, unsigned long long>), dim3(order.blocks),
+                           dim3(256), 0, s, g, N, boxlen, order, X, Y, Z, VX, VY, VZ);
 }
 
 // ---- displacement grids with a periodic z halo -------------------------------------
