@@ -20,27 +20,8 @@ namespace mitos {
 
 
 // ---- spectrum ------------------------------------------------------------------------
-inline double tophat_w(double x) {
-    if (x < 1e-3) return 1.0 - x * x / 10.0;
-    return 3.0 * (sin(x) - x * cos(x)) / (x * x * x);
-}
-
-// sigma_R^2 = int dk/(2 pi^2) k^2 P(k) W(kR)^2 with P = A k^n_s T_BBKS^2, Simpson in ln k
-inline double sigma8_amplitude(double n_s, double gamma, double sigma8, double R) {
-    const double lo = log(1e-6), hi = log(1e3);
-    const int n = 200000;
-    const double h = (hi - lo) / n;
-    double sum = 0.0;
-    for (int i = 0; i <= n; i++) {
-        const double k = exp(lo + i * h);
-        const double T = bbks_T(k, gamma);
-        const double W = tophat_w(k * R);
-        const double f = k * k * k * pow(k, n_s) * T * T * W * W / (2.0 * M_PI * M_PI);
-        const double w = (i == 0 || i == n) ? 1.0 : ((i & 1) ? 4.0 : 2.0);
-        sum += w * f;
-    }
-    return sigma8 * sigma8 / (sum * h / 3.0);
-}
+// A of P = A k^n_s T_BBKS^2 for sigma_R = sigma8 (sigma8.cpp)
+double sigma8_amplitude(double n_s, double gamma, double sigma8, double R);
 
 // Host: device table w[i] = 1/sinc(0.5 k_i boxlen/N)^order for i in [0, N),
 // k_i = freq_index(i)*2pi/boxlen.  The window of include/fft_kernels.h:198-219
