@@ -2,6 +2,7 @@
 // (include/distributed_grid.h:74-77, include/random.h:27-33, include/grf.h:30-31).
 #include <map>
 #include <mutex>
+#include <tuple>
 
 #include "../../include/mitos_hip.h"
 #include "api_util.h"
@@ -24,26 +25,27 @@ struct JumpEntry {
     int nbits;
 };
 
-int noise_jumps(int N, const Xo& s0, NoiseJumps* out) {
+int noise_jumps(int N, bool fp64, const Xo& s0, NoiseJumps* out) {
     static std::mutex mu;
-    static std::map<std::pair<int, int>, JumpEntry> cache;
+    static std::map<std::tuple<int, int, long>, JumpEntry> cache;
     int dev = 0;
     MITOS_HIP_CHECK(hipGetDevice(&dev));
-    const long H = N / 2 + 1;
-    const long rows = (long)N * N;
+    const long S = noise_segment(N, fp64);
+    const auto key = std::make_tuple(dev, N, S);
+    const long segs = ((long)N * N * (N / 2 + 1) + S - 1) / S;
     JumpEntry ent{nullptr, 0};
     {
         std::lock_guard<std::mutex> lock(mu);
-        auto it = cache.find(std::make_pair(dev, N));
+        auto it = cache.find(key);
         if (it != cache.end()) ent = it->second;
     }
     if (!ent.dev) {
         int nbits = 0;
-        while (nbits < 62 && (1L << nbits) < rows) nbits++;
+        while (nbits < 62 && (1L << nbits) < segs) nbits++;
         if (nbits == 0) nbits = 1;
         std::vector<uint64_t> tab((size_t)nbits * 1024);
         BitMat J;
-        bm_pow_step((uint64_t)(4 * H), J);
+        bm_pow_step((uint64_t)(4 * S), J);
         for (int b = 0; b < nbits; b++) {
             memcpy(&tab[(size_t)b * 1024], J.rows, sizeof(J.rows));
             if (b + 1 < nbits) bm_mul(J, J, J);
@@ -54,14 +56,12 @@ int noise_jumps(int N, const Xo& s0, NoiseJumps* out) {
                                   hipMemcpyHostToDevice));
         ent = JumpEntry{d, nbits};
         std::lock_guard<std::mutex> lock(mu);
-        cache[std::make_pair(dev, N)] = ent;
+        cache[key] = ent;
     }
     out->tab = ent.dev;
     out->nbits = ent.nbits;
-    out->s0 = s0;
-    Xo b = s0;
-    for (long i = 0; i < 4 * H - 4; i++) xo_next(b);
-    out->base = b;
+    out->base = s0;
+    for (int i = 0; i < 4; i++) xo_prev(out->base);
     return MITOS_OK;
 }
 
@@ -190,11 +190,11 @@ extern "C" int generate_complex_grf(struct distributed_grid* dg, rng_state* stat
     Xo s0;
     memcpy(s0.s, state->s, sizeof(s0.s));
     NoiseJumps J;
-    MITOS_TRY(set_last_error(noise_jumps(N, s0, &J)));
+    MITOS_TRY(set_last_error(noise_jumps(N, true, s0, &J)));
     hipStream_t s = api_stream();
     MITOS_TRY(set_last_error(launch_grf<double, AmpOne>(reinterpret_cast<cx<double>*>(dg->fbox),
-                                                        N / 2 + 1, N, dg->boxlen, 1, 0, J,
-                                                        AmpOne(), s)));
+                                                        N / 2 + 1, N, dg->boxlen, J, AmpOne(),
+                                                        s)));
     Xo s1 = s0;
     noise_advance(N, &s1);
     memcpy(state->s, s1.s, sizeof(s1.s));

@@ -7,16 +7,30 @@
 
 namespace mitos {
 
-// Per-grid-size jump data, resident on the device.
+// A thread draws a segment of consecutive modes of the half grid (in the dense
+// mode order): whole z-rows, or in FP64 below 256^3 pieces of 4 to 16 modes, where
+// one thread per row leaves most of the chip idle (64^3 has 4096 rows, 16
+// work-groups) and the correctly rounded normals make a long serial chain.  The
+// shorter the segments, the more start states; each size class has the length
+// that keeps about 10^5 threads.  generate_complex_grf, rows against segments: 64^3
+// 128 -> 54 us, 96^3 166 -> 68 us, 128^3 206 -> 102 us, 192^3 291 -> 201 us; at
+// 256^3 segments of 16 take 413 us, rows 388 us.  The FP32 draws are so short that a segment's
+// start state would cost more than it (the ensemble of 96: 54.6 -> 57.8 ms).
+inline int noise_segment(int N, bool fp64) {
+    return !fp64 || N >= 256 ? N / 2 + 1 : N > 160 ? 16 : N > 96 ? 8 : 4;
+}
+
+// Per-grid-size jump data, resident on the device; S = noise_segment.
 struct NoiseJumps {
-    const uint64_t* tab;  // nbits matrices J^(2^b), J = T^(4*(N/2+1)), 256*4 words each
+    const uint64_t* tab;  // nbits matrices J^(2^b), J = T^(4 S), 256*4 words each
     int nbits;
-    Xo s0;    // state before the first draw (row 0 starts here)
-    Xo base;  // state after 4*(N/2+1) - 4 draws (row 1 starts here)
+    // four draws before the first: the state of the stream with the DC mode's
+    // draws, which the reference does not take, so segment q starts at J^q base
+    Xo base;
 };
 
-// Host: jump data for grid size N starting from state s0 (table cached per N).
-int noise_jumps(int N, const Xo& s0, NoiseJumps* out);
+// Host: jump data for grid size N starting from state s0 (table cached).
+int noise_jumps(int N, bool fp64, const Xo& s0, NoiseJumps* out);
 // Host: state after the whole grid's draws, 4*(N*N*(N/2+1) - 1).
 int noise_advance(int N, Xo* st);
 
@@ -66,37 +80,31 @@ __device__ __forceinline__ uint64_t xo_next_dev(Xo& st) {
     return out;
 }
 
-// Start states of the 256 z-rows line0 + t of a 256-thread work-group (line0
+// Start states of the 256 segments line0 + t of a 256-thread work-group (line0
 // a multiple of 256), by the whole work-group.  A product M v of a jump
 // matrix and a state takes one parity per thread (output bit t = parity of
 // row t of M and v) and a ballot per wave (wave w holds word w).  The
-// work-group advances J.base to row line0 (the matrices of the bits of
-// line0 - 256 above bit 7, then J^255), then doubles: st[j + 2^k] =
-// J^(2^k) st[j] for k < 8, so thread t reads its row's state st[t].  That is
-// 255 + up to 20 products shared by 256 rows, against up to 20 per row when
-// every thread jumps on its own.  lds: 256 * 4 + 4 words.
+// work-group advances J.base to segment line0 (the matrices of the bits of line0,
+// all above bit 7), then doubles: st[j + 2^k] = J^(2^k) st[j] for k < 8, so thread
+// t reads its segment's state st[t].  That is 255 + up to 20 products shared by
+// 256 segments, against up to 20 per segment when every thread jumps on its own.
+// The products of a doubling are independent: four are in flight.  lds: 256 * 4 +
+// 4 words.
 __device__ __forceinline__ Xo block_row_start(const NoiseJumps& J, long line0, uint64_t* lds) {
     uint64_t(*st)[4] = reinterpret_cast<uint64_t(*)[4]>(lds);
     uint64_t* xw = lds + 256 * 4;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    auto apply = [&](int b, const Xo& v) -> Xo {
+    Xo v = J.base;
+    for (int b = 8; b < J.nbits; b++) {
+        if (!((line0 >> b) & 1)) continue;
         const uint64_t* row = J.tab + (size_t)b * 1024 + (size_t)t * 4;
         const uint64_t p = (row[0] & v.s[0]) ^ (row[1] & v.s[1]) ^ (row[2] & v.s[2]) ^
                            (row[3] & v.s[3]);
         const uint64_t w = __ballot(__builtin_popcountll(p) & 1);
         if (lane == 0) xw[wv] = w;
         __syncthreads();
-        const Xo r = {{xw[0], xw[1], xw[2], xw[3]}};
+        v = Xo{{xw[0], xw[1], xw[2], xw[3]}};
         __syncthreads();
-        return r;
-    };
-    Xo v = J.base;
-    if (line0 > 0) {
-        // row line0 starts after line0 - 1 jumps: (line0 - 256) + 255
-        const unsigned long hi = (unsigned long)(line0 - 256);
-        for (int b = 8; b < J.nbits; b++)
-            if ((hi >> b) & 1UL) v = apply(b, v);
-        for (int b = 0; b < 8; b++) v = apply(b, v);
     }
     if (t < 4) st[0][t] = v.s[t];
     __syncthreads();
@@ -104,19 +112,22 @@ __device__ __forceinline__ Xo block_row_start(const NoiseJumps& J, long line0, u
         const int m = 1 << k;
         const uint64_t* row = J.tab + (size_t)k * 1024 + (size_t)t * 4;
         const uint64_t r0 = row[0], r1 = row[1], r2 = row[2], r3 = row[3];
-        for (int j = 0; j < m; j++) {
-            const uint64_t p = (r0 & st[j][0]) ^ (r1 & st[j][1]) ^ (r2 & st[j][2]) ^
-                               (r3 & st[j][3]);
-            const uint64_t w = __ballot(__builtin_popcountll(p) & 1);
-            if (lane == 0) st[j + m][wv] = w;
+        for (int j0 = 0; j0 < m; j0 += 4) {
+            uint64_t p[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint64_t* s = st[j0 + j < m ? j0 + j : 0];
+                p[j] = (r0 & s[0]) ^ (r1 & s[1]) ^ (r2 & s[2]) ^ (r3 & s[3]);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint64_t w = __ballot(__builtin_popcountll(p[j]) & 1);
+                if (lane == 0 && j0 + j < m) st[j0 + j + m][wv] = w;
+            }
         }
         __syncthreads();
     }
-    // row 0 starts at s0 (the DC mode takes no draws); row line starts after
-    // line - 1 jumps from J.base
-    const int j = line0 > 0 ? t : t - 1;
-    Xo r = J.s0;
-    if (j >= 0) r = Xo{{st[j][0], st[j][1], st[j][2], st[j][3]}};
+    const Xo r = Xo{{st[t][0], st[t][1], st[t][2], st[t][3]}};
     __syncthreads();  // the table's reads precede the caller's reuse of lds
     return r;
 }
@@ -186,6 +197,26 @@ __host__ __device__ __forceinline__ void wavevec(int x, int y, int z, int N, dou
     k = sqrt(kx * kx + ky * ky + kz * kz);
 }
 
+// one mode: two normals times sqrt(L^3/2) = factor and the amplitude of n^2
+template <typename T, bool CR, typename AMP>
+__device__ __forceinline__ cx<T> grf_mode(Xo& gen, const AMP& amp, long n2, double factor) {
+    if constexpr (sizeof(T) == 4) {
+        const float ga = bm_normal_f(gen);
+        const float gb = bm_normal_f(gen);
+        float fm;
+        if constexpr (AMP::prescaled)
+            fm = amp.f(n2);  // (float)(factor * amp) made on the host
+        else
+            fm = (float)(factor * amp(n2));
+        return mk<T>(ga * fm, gb * fm);
+    } else {
+        const double a = bm_normal<CR>(gen) * factor;
+        const double b = bm_normal<CR>(gen) * factor;
+        const double m = amp(n2);
+        return mk<T>((T)(a * m), (T)(b * m));
+    }
+}
+
 // src/grf.c:26-69 with an amplitude amp(n2) applied to both parts (n2 =
 // integer |k|^2 / dk^2).  One thread walks one z-row in stream
 // order; a block's 256 rows are staged through LDS in chunks of 16 modes so
@@ -221,26 +252,14 @@ __global__ void __launch_bounds__(256)
                     stage[threadIdx.x * ZC + dz] = mk<T>(0, 0);
                     continue;
                 }
-                // the DC mode (n^2 = 0, k = 0) takes no draws
+                // the DC mode is zero; its place in the stream lies before the
+                // reference's first draw
                 const long n2 = n2xy + (long)z * z;
                 cx<T> val = mk<T>(0, 0);
-                if (n2 > 0) {
-                    if constexpr (sizeof(T) == 4) {
-                        const float ga = bm_normal_f(gen);
-                        const float gb = bm_normal_f(gen);
-                        float fm;
-                        if constexpr (AMP::prescaled)
-                            fm = amp.f(n2);  // (float)(factor * amp) made on the host
-                        else
-                            fm = (float)(factor * amp(n2));
-                        val = mk<T>(ga * fm, gb * fm);
-                    } else {
-                        const double a = bm_normal<CR>(gen) * factor;
-                        const double b = bm_normal<CR>(gen) * factor;
-                        const double m = amp(n2);
-                        val = mk<T>((T)(a * m), (T)(b * m));
-                    }
-                }
+                if (n2 > 0)
+                    val = grf_mode<T, CR>(gen, amp, n2, factor);
+                else
+                    for (int d = 0; d < 4; d++) (void)xo_next_dev(gen);
                 stage[threadIdx.x * ZC + dz] = val;
             }
         }
@@ -250,6 +269,85 @@ __global__ void __launch_bounds__(256)
             const int r = idx / ZC, dz = idx % ZC;
             const long l = line0 + r;
             if (l < nrows && z0 + dz < WZ) st(base + l * hs + z0 + dz, stage[r * ZC + dz]);
+        }
+        __syncthreads();
+    }
+}
+
+// k_grf with a segment of S modes per thread (grids below 256^3: the float
+// quotient of a mode index is within one of its row).  The work-group's modes are
+// consecutive; they are staged in LDS up to eight modes of every thread at a time
+// and stored as runs of that length.
+template <typename T, int S, typename AMP, bool CR>
+__global__ void __launch_bounds__(256)
+    k_grf_segments(cx<T>* out, long hs, int N, double boxlen, NoiseJumps J, AMP amp) {
+    constexpr int ZC = S < 8 ? S : 8;
+    static_assert(S % ZC == 0, "segments are whole chunks");
+    __shared__ __align__(16) cx<T> stage[256 * ZC > 1028 * 8 / (int)sizeof(cx<T>)
+                                             ? 256 * ZC
+                                             : 1028 * 8 / (int)sizeof(cx<T>)];
+    const int H = N / 2 + 1;
+    const unsigned modes = (unsigned)N * N * H;
+    const unsigned line0 = blockIdx.x * 256u;
+    Xo gen = block_row_start(J, (long)line0, reinterpret_cast<uint64_t*>(stage));
+    const double factor = sqrt(boxlen * boxlen * boxlen / 2);
+    const float invH = 1.0f / H;
+    // row and z' of a mode
+    auto split = [&](unsigned m, int& row, int& z) {
+        row = (int)((float)m * invH);
+        z = (int)m - row * H;
+        if (z < 0) {
+            row--;
+            z += H;
+        } else if (z >= H) {
+            row++;
+            z -= H;
+        }
+    };
+    const unsigned m0 = (line0 + threadIdx.x) * (unsigned)S;
+    int row, z;
+    split(m0, row, z);
+    int x = row / N, y = row - x * N;
+    int nx = freq_index(x, N), ny = freq_index(y, N), n2xy = nx * nx + ny * ny;
+    const int hz = (H + 15) / 16 * 16 < hs ? (H + 15) / 16 * 16 : (int)hs;
+    for (int c = 0; c < S; c += ZC) {
+        for (int d = 0; d < ZC; d++) {
+            const int n2 = n2xy + z * z;
+            cx<T> val = mk<T>(0, 0);
+            // the DC mode is zero; its place in the stream lies before the
+            // reference's first draw
+            if (m0 + c + d < modes) {
+                if (n2 > 0)
+                    val = grf_mode<T, CR>(gen, amp, n2, factor);
+                else
+                    for (int q = 0; q < 4; q++) (void)xo_next_dev(gen);
+            }
+            stage[threadIdx.x * ZC + d] = val;
+            if (++z == H) {
+                z = 0;
+                if (++y == N) {
+                    y = 0;
+                    x++;
+                }
+                nx = freq_index(x, N);
+                ny = freq_index(y, N);
+                n2xy = nx * nx + ny * ny;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ZC; i++) {
+            const unsigned idx = i * 256u + threadIdx.x;
+            const unsigned m = (line0 + idx / ZC) * (unsigned)S + c + idx % ZC;
+            if (m < modes) {
+                int r, zz;
+                split(m, r, zz);
+                cx<T>* dst = out + (long)r * hs;
+                st(dst + zz, stage[idx]);
+                // zeros in the row padding, up to the lines that hold modes
+                if (zz == H - 1)
+                    for (int q = H; q < hz; q++) st(dst + q, mk<T>(0, 0));
+            }
         }
         __syncthreads();
     }
@@ -302,12 +400,23 @@ struct AmpTableF {
 };
 
 template <typename T, typename AMP, bool CR = true>
-int launch_grf(cx<T>* out, long hs, int N, double boxlen, int nb, long bstride,
-               const NoiseJumps& J, AMP amp, hipStream_t s) {
+int launch_grf(cx<T>* out, long hs, int N, double boxlen, const NoiseJumps& J, AMP amp,
+               hipStream_t s) {
     const long rows = (long)N * N;
-    dim3 grid((unsigned)((rows + 255) / 256), nb);
-    hipLaunchKernelGGL((k_grf<T, AMP, CR>), grid, dim3(256), 0, s, out, hs, N, boxlen, bstride,
-                       J, amp);
+    if constexpr (sizeof(T) == 8) {
+        const int S = noise_segment(N, true);
+        if (S <= 16) {
+            const long segs = (rows * (N / 2 + 1) + S - 1) / S;
+            auto kern = S == 4   ? k_grf_segments<T, 4, AMP, CR>
+                        : S == 8 ? k_grf_segments<T, 8, AMP, CR>
+                                 : k_grf_segments<T, 16, AMP, CR>;
+            hipLaunchKernelGGL(kern, dim3((unsigned)((segs + 255) / 256)), dim3(256), 0, s, out,
+                               hs, N, boxlen, J, amp);
+            return hipGetLastError() == hipSuccess ? MITOS_OK : MITOS_ERR_DEVICE;
+        }
+    }
+    hipLaunchKernelGGL((k_grf<T, AMP, CR>), dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s,
+                       out, hs, N, boxlen, 0L, J, amp);
     return hipGetLastError() == hipSuccess ? MITOS_OK : MITOS_ERR_DEVICE;
 }
 

@@ -168,7 +168,7 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
     // 1. noise -> phi1(k), Hermitian planes (src/grf.c, src/2lpt.c:75)
     Xo s0 = xo_seed(cfg.seed);
     NoiseJumps J;
-    MITOS_TRY(noise_jumps(N, s0, &J));
+    MITOS_TRY(noise_jumps(N, sizeof(T) == 8, s0, &J));
     const double* amp = amp_tab ? amp_tab : phi1_table(N, L, amplitude, cfg.n_s, cfg.gamma);
     if (!amp) return MITOS_ERR_ALLOC;
     // FP64 keeps correctly rounded Box-Muller; FP32 rounds every value to float
@@ -184,11 +184,10 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
                 // same values as the double table's product)
                 const float* ampf = phi1_table_f(N, L, amplitude, cfg.n_s, cfg.gamma);
                 if (!ampf) return MITOS_ERR_ALLOC;
-                return launch_grf<T, AmpTableF, false>(K, hs, N, L, 1, 0, J, AmpTableF{ampf},
-                                                       s);
+                return launch_grf<T, AmpTableF, false>(K, hs, N, L, J, AmpTableF{ampf}, s);
             }
         }
-        return launch_grf<T, AmpTable, sizeof(T) == 8>(K, hs, N, L, 1, 0, J, AmpTable{amp}, s);
+        return launch_grf<T, AmpTable, sizeof(T) == 8>(K, hs, N, L, J, AmpTable{amp}, s);
     }));
     MITOS_TRY(timed(s, "hermitian_planes", 0.0,
                     [&] { return launch_hermitian<T>(K, hs, N, 1, 0, s); }));

@@ -38,6 +38,17 @@ __host__ __device__ __forceinline__ uint64_t xo_next(Xo& st) {
     return out;
 }
 
+// one step back: the state whose xo_next is st.  s3 and s0 follow from the rotation
+// and its xor; s1 ^ (s1 << 17) = s1' ^ s2' has the finite inverse sum of shifts
+inline void xo_prev(Xo& st) {
+    const uint64_t s3a = rotl64(st.s[3], 64 - 45);
+    const uint64_t s0 = st.s[0] ^ s3a;
+    const uint64_t z = st.s[1] ^ st.s[2];
+    const uint64_t s1 = z ^ (z << 17) ^ (z << 34) ^ (z << 51);
+    const uint64_t s2 = st.s[1] ^ s1 ^ s0;
+    st = Xo{{s0, s1, s2, s3a ^ s1}};
+}
+
 inline uint64_t splitmix64_next(uint64_t& x) {
     uint64_t r = x;
     x = r + 0x9E3779B97f4A7C15ULL;
