@@ -99,35 +99,30 @@ __global__ void __launch_bounds__(256)
         for (int j = 0; j < 4; j++) {
             const int qx = x0 + (int)(threadIdx.x >> 7) + 2 * j;
             const unsigned yz = (unsigned)qy * rs + zo;
-            // x1 = x0 - Sx(q), y1 = y0 - Fy(x1), z1 = z0 - Fz(x1, y1), with
+            // x1 = x0 - Sx(q), y1 = y0 - Fy(x1), z1 = z0 - Fz(x1, y1) as moves_s forms
+            // them: the cell of a particle at a cell's edge, and so its whole
+            // gradient, hangs on the last bit
+            T x1, y1, z1;
+            moves_s(sx, sy, sz, rs, N, sN, spacing, qx, qy, qz, x1, y1, z1);
             // dFy/dx, dFz/dx and dFz/dy from the same taps
-            const T x1 = (T)(qx * spacing) - sx[(unsigned)qx * plane + yz];
             int cx, cy;
             T wx[3], dwx[3], wy[3], dwy[3];
             unsigned ox[3], oy[3];
             tsc_axis_near_d(x1 * sN, cx, wx, dwx);
+            tsc_axis_near_d(y1 * sN, cy, wy, dwy);
             tap_rows(wrapf(cx, N, invN), N, plane, ox);
-            T y1 = (T)(qy * spacing), z1 = (T)(qz * spacing), fy = 0, Fy_x = 0;
+            tap_rows(wrapf(cy, N, invN), N, rs, oy);
+            T Fy_x = 0, Fz_x = 0, Fz_y = 0;
 #pragma unroll
             for (int a = 0; a < 3; a++) {
-                const T v = sy[ox[a] + yz];
-                fy += wx[a] * v;
-                Fy_x += dwx[a] * v;
-            }
-            y1 -= fy;
-            tsc_axis_near_d(y1 * sN, cy, wy, dwy);
-            tap_rows(wrapf(cy, N, invN), N, rs, oy);
-            T fz = 0, Fz_x = 0, Fz_y = 0;
-#pragma unroll
-            for (int a = 0; a < 3; a++)
+                Fy_x += dwx[a] * sy[ox[a] + yz];
 #pragma unroll
                 for (int b = 0; b < 3; b++) {
                     const T v = sz[ox[a] + oy[b] + zo];
-                    fz += wx[a] * wy[b] * v;
                     Fz_x += dwx[a] * wy[b] * v;
                     Fz_y += wx[a] * dwy[b] * v;
                 }
-            z1 -= fz;
+            }
             // CIC (analyse/src/mitos_read.c:285-320): d rho(corner) / d position
             int iX, iY, iZ;
             T dx, dy, dz;
@@ -241,10 +236,8 @@ __global__ void __launch_bounds__(512)
         tsc_axis_near(x1 * sN, cx[j], wx[j]);
         unsigned ox[3];
         tap_rows(wrapf(cx[j], N, invN), N, plane, ox);
-        T fy = 0;
-#pragma unroll
-        for (int a = 0; a < 3; a++) fy += wx[j][a] * sy[ox[a] + yz];
-        const T y1 = (T)(qy * spacing) - fy;
+        T y1 = (T)(qy * spacing);
+        y1 -= wx[j][0] * sy[ox[0] + yz] + wx[j][1] * sy[ox[1] + yz] + wx[j][2] * sy[ox[2] + yz];
         tsc_axis_near(y1 * sN, cy[j], wy[j]);
         sumx += cx[j] - qx;
         sumy += cy[j] - qy;

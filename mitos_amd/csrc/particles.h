@@ -1328,10 +1328,9 @@ __device__ __forceinline__ T wrap_pos(T x, T L) {
 // analyse/src/mitos_read.c:285-320 without the float position)
 template <typename T>
 __device__ __forceinline__ void cic_cell_t(T x, T icell, int N, int& i, T& d) {
-    const T X = x * icell;
-    T f = floor(X);
+    const T f = floor(x * icell);
     i = (int)f;
-    d = X - f;
+    d = fma(x, icell, -f);
     if (i >= N) {
         i -= N;
     }
@@ -1352,8 +1351,8 @@ __device__ __forceinline__ void adj_tile(unsigned b, int N, int& x0, int& y0, in
     x0 = (int)(b / (ntz * nty)) * kAdjTX;
 }
 
-// The adjoint's FP64 moves: positions in T (dense N^3 arrays) and their float
-// copies.
+// The adjoint's moves: float positions, and in FP64 the positions in T as well
+// (dense N^3 arrays).
 template <typename T>
 __global__ void __launch_bounds__(256)
     k_moves_s(const T* __restrict__ sx, const T* __restrict__ sy, const T* __restrict__ sz,
@@ -1377,13 +1376,15 @@ __global__ void __launch_bounds__(256)
         X[p] = (float)x;
         Y[p] = (float)y;
         Z[p] = (float)z;
-        xt[p] = x;
-        yt[p] = y;
-        zt[p] = z;
+        if constexpr (sizeof(T) == 8) {
+            xt[p] = x;
+            yt[p] = y;
+            zt[p] = z;
+        }
     }
 }
 
-// The adjoint's FP64 moves and deposit on grids without deposit tiles (N not a
+// The adjoint's moves and deposit on grids without deposit tiles (N not a
 // multiple of 32): positions kept in T for the deposit (their float copies go
 // to X/Y/Z), fixed-point weights 2^-shift with global atomics (order
 // independent).
@@ -1472,13 +1473,19 @@ __device__ __forceinline__ void cic_axis_f(float x, float cell, float cinv, int 
 // for the tiled deposit: base cell q + r with r the periodic cell offset in
 // [-N/2, N/2) (so the base index lies in [-N/2, 3N/2)), and the in-cell
 // offsets.
-template <typename W, typename P>
+// CT: the cells of the adjoint's forward (cic_cell_t, positions in [0, L)).
+template <typename W, bool CT = false, typename P>
 __device__ __forceinline__ void cic_lattice_cell(P x, P y, P z, int N, double boxlen,
                                                  float cell, float cinv, int qx, int qy, int qz,
                                                  int& rx, int& ry, int& rz, W& fx, W& fy,
                                                  W& fz) {
     int iX, iY, iZ;
-    if constexpr (sizeof(W) == 8) {
+    if constexpr (CT) {
+        const W sN = (W)(N / boxlen);
+        cic_cell_t((W)x, sN, N, iX, fx);
+        cic_cell_t((W)y, sN, N, iY, fy);
+        cic_cell_t((W)z, sN, N, iZ, fz);
+    } else if constexpr (sizeof(W) == 8) {
         cic_cell(x, y, z, N, boxlen, iX, iY, iZ, fx, fy, fz);
     } else {
         cic_axis_f(x, cell, cinv, N, iX, fx);
@@ -1573,7 +1580,7 @@ __device__ __noinline__ inline void cic_list_carry(const CicLists& l, unsigned m
 // pipeline), 32-bit window with carries.
 // PT: type of the positions (double: the FP64 adjoint's)
 template <typename W, int PX, int PY, int PZ, int RX, int RY, int RZ, int NT,
-          bool STREAM = false, typename PT = float>
+          bool STREAM = false, typename PT = float, bool CT = false>
 __global__ void __launch_bounds__(NT)
     k_cic_lattice(const PT* __restrict__ X, const PT* __restrict__ Y,
                   const PT* __restrict__ Z, int N, double boxlen, unsigned long long* grid,
@@ -1625,7 +1632,7 @@ __global__ void __launch_bounds__(NT)
         for (int i = 0; i < K; i++) {
             const int p = threadIdx.x + NT * i;
             const int lz = p % PZ, ly = (p / PZ) % PY, lx = p / (PZ * PY);
-            cic_lattice_cell(px[i], py[i], pz[i], N, boxlen, cell, cinv, tx * PX + lx,
+            cic_lattice_cell<W, CT>(px[i], py[i], pz[i], N, boxlen, cell, cinv, tx * PX + lx,
                              ty * PY + ly, tz * PZ + lz, rxs[i], rys[i], rzs[i], fx[i], fy[i],
                              fz[i]);
             sx += rxs[i];
@@ -1782,8 +1789,8 @@ __global__ void __launch_bounds__(NT)
             const unsigned idx = ((unsigned)qx * N + (unsigned)qy) * N + qz;
             int rx, ry, rz;
             W dx, dy, dz;
-            cic_lattice_cell(X[idx], Y[idx], Z[idx], N, boxlen, cell, cinv, qx, qy, qz, rx, ry,
-                             rz, dx, dy, dz);
+            cic_lattice_cell<W, CT>(X[idx], Y[idx], Z[idx], N, boxlen, cell, cinv, qx, qy, qz,
+                                    rx, ry, rz, dx, dy, dz);
             unsigned long long w[8];
             cic_weights(dx, dy, dz, w);
             cic_global_near(grid, N, qx + rx, qy + ry, qz + rz, w);
@@ -1895,7 +1902,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8)))
 }
 
 // Third pass: far particles and window carries added to the grid.
-template <typename W>
+template <typename W, bool CT>
 __global__ void __launch_bounds__(256)
     k_cic_far(const float* __restrict__ X, const float* __restrict__ Y,
               const float* __restrict__ Z, int N, double boxlen, unsigned long long* grid,
@@ -1910,8 +1917,8 @@ __global__ void __launch_bounds__(256)
                   qx = (int)(idx / ((unsigned)N * (unsigned)N));
         int rx, ry, rz;
         W dx, dy, dz;
-        cic_lattice_cell(X[idx], Y[idx], Z[idx], N, boxlen, cell, cinv, qx, qy, qz, rx, ry, rz,
-                         dx, dy, dz);
+        cic_lattice_cell<W, CT>(X[idx], Y[idx], Z[idx], N, boxlen, cell, cinv, qx, qy, qz, rx,
+                                ry, rz, dx, dy, dz);
         unsigned long long w[8];
         cic_weights(dx, dy, dz, w);
         cic_global_near(grid, N, qx + rx, qy + ry, qz + rz, w);
@@ -1921,9 +1928,10 @@ __global__ void __launch_bounds__(256)
 }
 
 // the tile kernel of window type W
-template <typename W, bool STREAM = false, typename PT = float, typename C = CicTile<W>>
+template <typename W, bool STREAM = false, typename PT = float, bool CT = false,
+          typename C = CicTile<W>>
 constexpr auto cic_lattice_kernel() {
-    return k_cic_lattice<W, C::PX, C::PY, C::PZ, C::RX, C::RY, C::RZ, C::NT, STREAM, PT>;
+    return k_cic_lattice<W, C::PX, C::PY, C::PZ, C::RX, C::RY, C::RZ, C::NT, STREAM, PT, CT>;
 }
 
 static __global__ void k_zero_i32(int* p, int n) {
@@ -1981,7 +1989,7 @@ inline CicLists cic_lists(int N, void* ws, void* lists_mem) {
 // the windows go to ws, far particles and carries to the lists, and
 // cic_gather_launch then cic_far_launch write the grid, which need not be
 // cleared.  Otherwise the windows are added to a cleared grid with atomics.
-template <typename W, bool STREAM, typename PT = float>
+template <typename W, bool STREAM, typename PT = float, bool CT = false>
 inline int cic_lattice_launch(const PT* X, const PT* Y, const PT* Z, int N,
                               double boxlen, unsigned long long* grid, void* ws,
                               void* lists_mem, hipStream_t s) {
@@ -2002,7 +2010,7 @@ inline int cic_lattice_launch(const PT* X, const PT* Y, const PT* Z, int N,
             MITOS_HIP_CHECK(
                 hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
             MITOS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per, cic_lattice_kernel<W, STREAM, PT>(), C::NT, 0));
+                &per, cic_lattice_kernel<W, STREAM, PT, CT>(), C::NT, 0));
             if (cus <= 0 || per <= 0) return MITOS_ERR_DEVICE;
             it = resident.emplace(dev, cus * per).first;
         }
@@ -2021,7 +2029,7 @@ inline int cic_lattice_launch(const PT* X, const PT* Y, const PT* Z, int N,
         // mean-offset maxima (meta[0..2]) and list counts (meta[4..5]) start at 0
         hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, meta, 8);
     }
-    hipLaunchKernelGGL((cic_lattice_kernel<W, STREAM, PT>()), dim3(groups), dim3(C::NT), 0, s, X, Y,
+    hipLaunchKernelGGL((cic_lattice_kernel<W, STREAM, PT, CT>()), dim3(groups), dim3(C::NT), 0, s, X, Y,
                        Z, N, boxlen, grid, ntiles, scratch, means, meta, lists);
     return MITOS_OK;
 }
@@ -2042,11 +2050,11 @@ inline int cic_gather_launch(int N, unsigned long long* grid, void* ws, hipStrea
 }
 
 // third pass of the two-pass deposit: far particles and carries
-template <typename W>
+template <typename W, bool CT = false>
 inline int cic_far_launch(const float* X, const float* Y, const float* Z, int N, double boxlen,
                           unsigned long long* grid, void* ws, void* lists_mem, hipStream_t s) {
     if (!ws || !lists_mem || cic_stream_bytes<W>(N) == 0) return MITOS_ERR_ARG;
-    hipLaunchKernelGGL((k_cic_far<W>), dim3(1024), dim3(256), 0, s, X, Y, Z, N, boxlen, grid,
+    hipLaunchKernelGGL((k_cic_far<W, CT>), dim3(1024), dim3(256), 0, s, X, Y, Z, N, boxlen, grid,
                        cic_lists<W>(N, ws, lists_mem));
     return MITOS_OK;
 }

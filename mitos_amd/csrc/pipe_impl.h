@@ -306,10 +306,7 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
         // grid cell, the one-pass and the adjoint-mode deposits add to a
         // cleared grid (far-particle lists use K, free after combine_x)
         typedef typename std::conditional<sizeof(T) == 4, float, double>::type M;
-        // the FP64 adjoint's forward keeps its positions in double up to the
-        // deposit; in FP32 the positions are the particle arrays
-        const bool keep_t = noise_in && sizeof(T) == 8;
-        const bool two_pass = !keep_t && cic_ws && NN % 32 == 0 && Ml == NN &&
+        const bool two_pass = cic_ws && NN % 32 == 0 && Ml == NN &&
                               cic_list_bytes<M>(NN) <= sizeof(cx<T>) * (size_t)csize;
         if (!two_pass)
             MITOS_TRY(timed(s, "cic_clear", 8.0 * np, [&] {
@@ -319,23 +316,33 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
             }));
         mark(5);
         // FP32 moves the particles in float arithmetic, FP64 in double
-        if (keep_t) {
+        if (noise_in) {
+            // the forward of the adjoint: the moves and cells that its backward
+            // differentiates, positions in T up to the deposit.  FP64 positions lie
+            // in the A grids (free once the displacement grids are made).
             MITOS_TRY(timed(s, "move_deposit", 3 * Rg + 12.0 * np + 8.0 * np, [&] {
-                if constexpr (sizeof(T) == 8) {
-                    if (NN % 32 == 0) {
-                        // positions into the A grids (free once the displacement
-                        // grids are made), then the tiled LDS deposit: 0.06 ms at
-                        // 96^3, a global atomic per corner and particle 0.30 ms
-                        T* xt = reinterpret_cast<T*>(a(0));
-                        T* yt = reinterpret_cast<T*>(a(1));
-                        T* zt = reinterpret_cast<T*>(a(2));
-                        hipLaunchKernelGGL((k_moves_s<T>), dim3(adj_tiles(NN)), dim3(256), 0, s,
-                                           psi(0), psi(1), psi(2), (unsigned)(prs()), NN, L,
-                                           spacing, X, Y, Z, xt, yt, zt);
-                        MITOS_TRY((cic_lattice_launch<M, false, T>(xt, yt, zt, NN, L, cic(),
-                                                                   nullptr, nullptr, s)));
-                        return launch_status();
+                if constexpr (NN % 32 == 0) {
+                    // moves, then the tiled LDS deposit of the pipeline: 0.06 ms at
+                    // 96^3 in FP64, a global atomic per corner and particle 0.30 ms
+                    T* xt = reinterpret_cast<T*>(a(0));
+                    T* yt = reinterpret_cast<T*>(a(1));
+                    T* zt = reinterpret_cast<T*>(a(2));
+                    hipLaunchKernelGGL((k_moves_s<T>), dim3(adj_tiles(NN)), dim3(256), 0, s,
+                                       psi(0), psi(1), psi(2), (unsigned)(prs()), NN, L, spacing,
+                                       X, Y, Z, xt, yt, zt);
+                    if constexpr (sizeof(T) == 8) {
+                        MITOS_TRY((cic_lattice_launch<M, false, T, true>(
+                            xt, yt, zt, NN, L, cic(), nullptr, nullptr, s)));
+                    } else if (two_pass) {
+                        MITOS_TRY((cic_lattice_launch<M, true, float, true>(
+                            X, Y, Z, NN, L, cic(), cic_ws, K, s)));
+                        MITOS_TRY(cic_gather_launch<M>(NN, cic(), cic_ws, s));
+                        MITOS_TRY((cic_far_launch<M, true>(X, Y, Z, NN, L, cic(), cic_ws, K, s)));
+                    } else {
+                        MITOS_TRY((cic_lattice_launch<M, false, float, true>(
+                            X, Y, Z, NN, L, cic(), nullptr, nullptr, s)));
                     }
+                    return launch_status();
                 }
                 hipLaunchKernelGGL((k_move_deposit_s<T>), dim3(nblk(np)), dim3(256), 0, s,
                                    psi(0), psi(1), psi(2), (unsigned)(prs()),
