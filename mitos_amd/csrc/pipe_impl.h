@@ -354,16 +354,13 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
             MITOS_TRY(timed(s, "displace_tsc", 3 * Rg + 12.0 * nl, [&] {
                 constexpr int NT = NN >= 256 ? 256 : 64;
                 const int nch = (NN + NT - 1) / NT;
-                const dim3 grid((unsigned)((long)NN * NN * nch));
                 const unsigned rs = (unsigned)(prs());
                 if (Ml != NN) {
                     // an M^3 lattice off the grid nodes: the 27-tap moves
                     // at each particle's position
-                    const int nchm = (Ml + NT - 1) / NT;
-                    hipLaunchKernelGGL((k_displace_lattice<T, M, NT>),
-                                       dim3((unsigned)((long)Ml * Ml * nchm)), dim3(NT), 0, s,
-                                       psi(0), psi(1), psi(2), rs, NN, Ml, nchm, L, spacing,
-                                       X, Y, Z);
+                    hipLaunchKernelGGL((k_displace_lattice<T, M>),
+                                       dim3(displace_lattice_blocks(Ml)), dim3(256), 0, s,
+                                       psi(0), psi(1), psi(2), rs, NN, Ml, L, spacing, X, Y, Z);
                 } else if (STENCIL && NN % 16 == 0 && tsc_tile) {
                     auto tile = [&](auto kern, int txn, int ty, int tz, int pp) {
                         const dim3 gridt(
@@ -407,9 +404,9 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
                     tile(k_displace_tile_ref<8, 8, 16, 4, 256, 8>, 8, 8, 16, 4);
                   }
                 } else {
-                    hipLaunchKernelGGL((k_displace_lattice<T, M, NT>), grid, dim3(NT), 0, s,
-                                       psi(0), psi(1), psi(2), rs, NN, NN, nch, L, spacing,
-                                       X, Y, Z);
+                    hipLaunchKernelGGL((k_displace_lattice<T, M>),
+                                       dim3(displace_lattice_blocks(NN)), dim3(256), 0, s,
+                                       psi(0), psi(1), psi(2), rs, NN, NN, L, spacing, X, Y, Z);
                 }
                 return launch_status();
             }));
