@@ -50,7 +50,36 @@ struct MultiK<T, L, AXIS, DIR, NIN, CODES, Radices<Rs...>> {
     }
 };
 
-template <typename T, int N, typename RAD = typename LineCfgS<N / 2>::R>
+// Lines of k_hess_z: in FP64 four values a thread for powers of two, so the four
+// arrays of a thread's row leave room for its addresses and twiddles, and a row of
+// 256 is one wave, whose barriers wait on nobody (rows of fewer threads share a
+// wave).  Against eight a thread: 512^3 3.05 -> 2.14 ms, the drop-in 2LPT at 256^3
+// 1.80 -> 1.70 ms.  Bound by latency at two waves a SIMD: four waves (addresses and
+// twiddles formed anew per row) took 2.33 ms at 512^3 and 1.80 ms.
+template <typename T, int L>
+struct HessCfg : LineCfgS<L> {};
+template <>
+struct HessCfg<double, 64> {
+    static constexpr int E = 4;
+    typedef Radices<4, 4, 4> R;
+};
+template <>
+struct HessCfg<double, 128> {
+    static constexpr int E = 4;
+    typedef Radices<4, 4, 4, 2> R;
+};
+template <>
+struct HessCfg<double, 256> {
+    static constexpr int E = 4;
+    typedef Radices<4, 4, 4, 4> R;
+};
+template <>
+struct HessCfg<double, 512> {
+    static constexpr int E = 4;
+    typedef Radices<4, 4, 4, 4, 2> R;
+};
+
+template <typename T, int N, typename RAD = typename HessCfg<T, N / 2>::R>
 struct HessZK;
 template <typename T, int N, int... Rs>
 struct HessZK<T, N, Radices<Rs...>> {
@@ -59,11 +88,13 @@ struct HessZK<T, N, Radices<Rs...>> {
     static int go(const MultiPtrs<T, 6, 1>& P, long hs, double dk, T scale, T* real, long rs,
                   hipStream_t s, long nrows = (long)N * N) {
         constexpr int L = N / 2;
-        constexpr int E = LineCfgS<L>::E;
+        constexpr int E = HessCfg<T, L>::E;
         constexpr int TPL = L / E;
         // a row of a wave or more: one row per work-group (no barrier waits
         // on other rows' waves)
-        constexpr int RW = TPL >= 64 ? 1 : RowsPerBlock<TPL>::value;
+        constexpr int RW = TPL >= 64                            ? 1
+                           : sizeof(T) == 8 && E == 4 && TPL >= 16 ? 64 / TPL
+                                                   : RowsPerBlock<TPL>::value;
         const cx<T>* tw = twiddles<T>(L);
         const cx<T>* twN = twiddles<T>(N);
         if (!tw || !twN) return MITOS_ERR_ALLOC;
