@@ -265,8 +265,10 @@ __global__ void __launch_bounds__(512)
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         if (!ok) continue;
-        const int ax = cx[j] - 1 - wx0, ay = cy[j] - 1 - wy0;
-        const bool inx = ax >= 0 && ax + 2 < WX, in = inx && ay >= 0 && ay + 2 < WX;
+        // unsigned: a cell anywhere in the int range falls out of the window
+        const unsigned ax = (unsigned)cx[j] - 1u - (unsigned)wx0;
+        const unsigned ay = (unsigned)cy[j] - 1u - (unsigned)wy0;
+        const bool inx = ax < WX - 2u, in = inx && ay < WX - 2u;
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             const unsigned long long vy =

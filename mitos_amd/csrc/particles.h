@@ -85,16 +85,25 @@ __device__ __forceinline__ void tsc_axis_short(double X, int& i0, double w[3]) {
     w[2] = ok ? 0.5 * r * r : 0;
 }
 
-__device__ __forceinline__ int wrapi(int i, int N) { return ((i % N) + N) % N; }
+__host__ __device__ __forceinline__ int wrapi(int i, int N) { return ((i % N) + N) % N; }
 // wrap of an index known to lie in [-N, 2N)
-__device__ __forceinline__ int wrap1(int i, int N) { return i < 0 ? i + N : (i >= N ? i - N : i); }
+__host__ __device__ __forceinline__ int wrap1(int i, int N) {
+    return i < 0 ? i + N : (i >= N ? i - N : i);
+}
 
-// periodic wrap of any int index (floor division through a float reciprocal,
-// then one correction each way; exact for |i| < 2^22)
-__device__ __forceinline__ int wrapf(int i, int N, float invN) {
+// periodic wrap of an index |i| < 2^22 (floor division through a float
+// reciprocal, then one correction each way).  Past that the quotient is off by
+// more than one and the value may lie outside [0, N).
+__host__ __device__ __forceinline__ int wrapf_near(int i, int N, float invN) {
     int r = i - N * (int)floorf((float)i * invN);
     r = r < 0 ? r + N : r;
     return r >= N ? r - N : r;
+}
+// wrapf_near kept inside the grid for any int: 2^22 cells from the box a float
+// position no longer resolves its cell, but its taps are read all the same
+__host__ __device__ __forceinline__ int wrapf(int i, int N, float invN) {
+    const int r = wrapf_near(i, N, invN);
+    return r < 0 ? 0 : (r < N ? r : N - 1);
 }
 
 // gridTSC_dg (src/grids_interp.c:267-309) on one rank: all taps wrap
@@ -113,7 +122,7 @@ __device__ __forceinline__ TscTaps<O> tsc_taps(double X, int N, float invN, O st
     TscTaps<O> t;
     int i0;
     tsc_axis_short(X, i0, t.w);
-    int b = wrapf(i0, N, invN);
+    int b = wrapf_near(i0, N, invN);
     if ((unsigned)b >= (unsigned)N) b = wrapi(i0, N);  // far outside the box
 #pragma unroll
     for (int k = 0; k < 3; k++) t.o[k] = (O)wrap1(b + k, N) * stride;
@@ -1016,6 +1025,7 @@ __global__ void __launch_bounds__(TXN / PP * TY * TZ) __attribute__((amdgpu_wave
     // stage window rows 0 .. nrow - 1 of src, nyr rows per x, from (xs, ys)
     auto stage = [&](const double* __restrict__ src, int nrow, int nyr, int xs, int ys) {
         const float rcp = 1.0f / (float)nyr;
+        const int xw = wrapf(xs, N, invN), yw = wrapf(ys, N, invN);
         for (int r0 = rg; r0 < nrow; r0 += RG * U) {
             double v[U];
 #pragma unroll
@@ -1032,8 +1042,8 @@ __global__ void __launch_bounds__(TXN / PP * TY * TZ) __attribute__((amdgpu_wave
                         xi++;
                         yi -= nyr;
                     }
-                    const unsigned o = (unsigned)wrapf(xs + xi, N, invN) * plane +
-                                       (unsigned)wrapf(ys + yi, N, invN) * rs +
+                    const unsigned o = (unsigned)wrapf_near(xw + xi, N, invN) * plane +
+                                       (unsigned)wrapf_near(yw + yi, N, invN) * rs +
                                        (unsigned)(MITOS_PSI_HO - 1 + z0 + rl);
                     v[u] = src[o];
                 }

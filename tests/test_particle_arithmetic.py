@@ -1,0 +1,39 @@
+"""The index and weight arithmetic of the particle kernels, compiled for the host:
+positions far from the box, at the edges of cells and of the box."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("host_checks") / "particles.so")
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-std=c++20", "-O1", "-fPIC",
+                    "-ffp-contract=off", "-shared", "-o", out,
+                    os.path.join(HERE, "host_checks", "particles.cpp")],
+                   check=True, capture_output=True)
+    return ctypes.CDLL(out)
+
+
+def _p(a):
+    return a.ctypes.data_as(ctypes.c_void_p)
+
+
+# every compiled grid size: powers of two, whose reciprocal is exact, and 3 * 2^k
+@pytest.mark.parametrize("N", [8, 16, 24, 48, 96, 256, 384, 1024, 1536])
+def test_wrapped_cells_stay_in_the_grid(host, N):
+    rng = np.random.default_rng(N)
+    near = rng.integers(-(1 << 22) + 1, 1 << 22, 200000)
+    far = rng.integers(-(1 << 31), 1 << 31, 200000)
+    ends = np.array([0, -1, N, N - 1, -N, -(1 << 31), (1 << 31) - 1])
+    i = np.concatenate([near, far, ends]).astype(np.int32)
+    out = np.empty_like(i)
+    host.check_wrapf(N, ctypes.c_long(i.size), _p(i), _p(out))
+    assert out.min() >= 0 and out.max() < N
+    assert np.array_equal(out[:near.size], np.mod(near, N))
