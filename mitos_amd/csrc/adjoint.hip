@@ -124,15 +124,12 @@ __global__ void __launch_bounds__(256)
                 }
             }
             // CIC (analyse/src/mitos_read.c:285-320): d rho(corner) / d position
-            int iX, iY, iZ;
+            int cx0, cy0, cz0;
             T dx, dy, dz;
-            cic_cell_t(wrap_pos(x1, Lb), sN, N, iX, dx);
-            cic_cell_t(wrap_pos(y1, Lb), sN, N, iY, dy);
-            cic_cell_t(wrap_pos(z1, Lb), sN, N, iZ, dz);
-            auto wrapped = [&](int i) { return (unsigned)i < (unsigned)N ? i : wrapi(i, N); };
-            const int cx0 = wrapped(iX), cxp = wrap1(cx0 + 1, N);
-            const int cy0 = wrapped(iY), cyp = wrap1(cy0 + 1, N);
-            const int cz0 = wrapped(iZ), czp = wrap1(cz0 + 1, N);
+            cic_cell_t(wrap_pos(x1, Lb), sN, N, cx0, dx);
+            cic_cell_t(wrap_pos(y1, Lb), sN, N, cy0, dy);
+            cic_cell_t(wrap_pos(z1, Lb), sN, N, cz0, dz);
+            const int cxp = wrap1(cx0 + 1, N), cyp = wrap1(cy0 + 1, N), czp = wrap1(cz0 + 1, N);
             auto g = [&](int a, int b, int c) { return grho[((size_t)a * N + b) * N + c]; };
             const T g000 = g(cx0, cy0, cz0), g100 = g(cxp, cy0, cz0), g010 = g(cx0, cyp, cz0),
                     g001 = g(cx0, cy0, czp), g110 = g(cxp, cyp, cz0), g101 = g(cxp, cy0, czp),

@@ -1323,9 +1323,10 @@ __device__ __forceinline__ void moves_s(const T* __restrict__ sx, const T* __res
     z -= d;
 }
 
-// periodic wrap of a coordinate in T (exact subtractions for |x| < L)
+// periodic wrap of a coordinate in T (exact subtractions for |x| < L; many box
+// lengths away x - L floor(x / L) is inexact and may stay outside [0, L))
 template <typename T>
-__device__ __forceinline__ T wrap_pos(T x, T L) {
+__host__ __device__ __forceinline__ T wrap_pos(T x, T L) {
     if (x < 0) x += L;
     if (x >= L) x -= L;
     if (x < 0 || x >= L) x = x - L * floor(x / L);
@@ -1333,15 +1334,14 @@ __device__ __forceinline__ T wrap_pos(T x, T L) {
 }
 
 // CIC cell and weights of a position in T (the cell offsets of
-// analyse/src/mitos_read.c:285-320 without the float position)
+// analyse/src/mitos_read.c:285-320 without the float position).  The cell lies in
+// [0, N) for any position: wrap_pos does not bring every one into the box.
 template <typename T>
-__device__ __forceinline__ void cic_cell_t(T x, T icell, int N, int& i, T& d) {
+__host__ __device__ __forceinline__ void cic_cell_t(T x, T icell, int N, int& i, T& d) {
     const T f = floor(x * icell);
     i = (int)f;
     d = fma(x, icell, -f);
-    if (i >= N) {
-        i -= N;
-    }
+    i = (unsigned)i < (unsigned)N ? i : wrapi(i, N);
 }
 
 // Lattice site of thread t's particle j in the order of the adjoint's particle
@@ -1481,9 +1481,9 @@ __device__ __forceinline__ void cic_axis_f(float x, float cell, float cinv, int 
 // for the tiled deposit: base cell q + r with r the periodic cell offset in
 // [-N/2, N/2) (so the base index lies in [-N/2, 3N/2)), and the in-cell
 // offsets.
-// CT: the cells of the adjoint's forward (cic_cell_t, positions in [0, L)).
+// CT: the cells of the adjoint's forward (cic_cell_t).
 template <typename W, bool CT = false, typename P>
-__device__ __forceinline__ void cic_lattice_cell(P x, P y, P z, int N, double boxlen,
+__host__ __device__ __forceinline__ void cic_lattice_cell(P x, P y, P z, int N, double boxlen,
                                                  float cell, float cinv, int qx, int qy, int qz,
                                                  int& rx, int& ry, int& rz, W& fx, W& fy,
                                                  W& fz) {

@@ -12,4 +12,26 @@ void check_wrapf(int N, long n, const int* i, int* out) {
     for (long k = 0; k < n; k++) out[k] = wrapf(i[k], N, 1.0f / N);
 }
 
+// the deposit's base index (site + periodic offset) of positions along one axis
+void check_lattice_cell_f(int N, double L, long n, int site, const float* x, int* base) {
+    for (long k = 0; k < n; k++) {
+        const float p = wrap_pos(x[k], (float)L);
+        int rx, ry, rz;
+        float fx, fy, fz;
+        cic_lattice_cell<float, true>(p, p, p, N, L, 0.0f, 0.0f, site, site, site, rx, ry, rz, fx,
+                                      fy, fz);
+        base[k] = site + rx;
+    }
+}
+void check_lattice_cell_d(int N, double L, long n, int site, const double* x, int* base) {
+    for (long k = 0; k < n; k++) {
+        const double p = wrap_pos(x[k], L);
+        int rx, ry, rz;
+        double fx, fy, fz;
+        cic_lattice_cell<double, true>(p, p, p, N, L, 0.0f, 0.0f, site, site, site, rx, ry, rz,
+                                       fx, fy, fz);
+        base[k] = site + rx;
+    }
+}
+
 }  // extern "C"

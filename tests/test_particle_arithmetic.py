@@ -37,3 +37,20 @@ def test_wrapped_cells_stay_in_the_grid(host, N):
     host.check_wrapf(N, ctypes.c_long(i.size), _p(i), _p(out))
     assert out.min() >= 0 and out.max() < N
     assert np.array_equal(out[:near.size], np.mod(near, N))
+
+
+# the deposit takes a base index in [-N, 2N) and wraps it once: positions up to far
+# more box lengths than a float resolves, infinities and NaN
+@pytest.mark.parametrize("N,L", [(32, 48.0), (96, 1000 / 3), (256, 500.0), (256, 512.0)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_deposit_cells_stay_in_the_grid(host, N, L, dtype):
+    rng = np.random.default_rng(N)
+    scale = 10.0 ** rng.uniform(0, 30, 200000)
+    x = np.concatenate([L * scale * rng.choice([-1, 1], scale.size), L * rng.random(200000),
+                        [0, L, np.nextafter(dtype(L), dtype(0)), -1e-30, np.inf, -np.inf, np.nan]])
+    x = x.astype(dtype)
+    base = np.empty(x.size, np.int32)
+    check = host.check_lattice_cell_f if dtype == np.float32 else host.check_lattice_cell_d
+    for site in (0, N // 2, N - 1):
+        check(N, ctypes.c_double(L), ctypes.c_long(x.size), site, _p(x), _p(base))
+        assert base.min() >= -N and base.max() < 2 * N
