@@ -1188,8 +1188,8 @@ __device__ __forceinline__ void cic_cell(P X, P Y, P Z, int N, double boxlen, in
     dz = Zc - iZ;
 }
 
-__device__ __forceinline__ void cic_weights(double dx, double dy, double dz,
-                                            unsigned long long w[8]) {
+__host__ __device__ __forceinline__ void cic_weights(double dx, double dy, double dz,
+                                                     unsigned long long w[8]) {
 #pragma clang fp contract(off)
     const double tx = 1.0 - dx, ty = 1.0 - dy, tz = 1.0 - dz;
     const double S = (double)(1ULL << MITOS_CIC_SHIFT);
@@ -1237,8 +1237,8 @@ __device__ __forceinline__ void cic_cell_f(float X, float Y, float Z, int N, flo
     dz = D[2];
 }
 
-__device__ __forceinline__ void cic_weights(float dx, float dy, float dz,
-                                            unsigned long long w[8]) {
+__host__ __device__ __forceinline__ void cic_weights(float dx, float dy, float dz,
+                                                     unsigned long long w[8]) {
     const float tx = 1.0f - dx, ty = 1.0f - dy, tz = 1.0f - dz;
     const float S = (float)(1u << MITOS_CIC_SHIFT_F32);
     const float a = tx * ty, b = dx * ty, c = tx * dy, d = dx * dy;
@@ -1335,12 +1335,16 @@ __host__ __device__ __forceinline__ T wrap_pos(T x, T L) {
 
 // CIC cell and weights of a position in T (the cell offsets of
 // analyse/src/mitos_read.c:285-320 without the float position).  The cell lies in
-// [0, N) for any position: wrap_pos does not bring every one into the box.
+// [0, N) for any position: wrap_pos does not bring every one into the box.  Where
+// the product rounds up to the next cell's edge the offset from there is negative
+// by that rounding: zero, so that no weight is negative and a particle's eight sum
+// to one (the deposit and its adjoint share the offset; a NaN stays).
 template <typename T>
 __host__ __device__ __forceinline__ void cic_cell_t(T x, T icell, int N, int& i, T& d) {
     const T f = floor(x * icell);
     i = (int)f;
-    d = fma(x, icell, -f);
+    const T r = fma(x, icell, -f);
+    d = r < 0 ? (T)0 : (r > 1 ? (T)1 : r);
     i = (unsigned)i < (unsigned)N ? i : wrapi(i, N);
 }
 

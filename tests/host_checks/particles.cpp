@@ -34,4 +34,18 @@ void check_lattice_cell_d(int N, double L, long n, int site, const double* x, in
     }
 }
 
+// in-cell offset of positions along one axis, and the fixed-point mass of a
+// particle with that offset on all three
+void check_cell_mass(int N, double L, long n, const float* x, float* d,
+                     unsigned long long* mass) {
+    for (long k = 0; k < n; k++) {
+        int i;
+        cic_cell_t(wrap_pos(x[k], (float)L), (float)(N / L), N, i, d[k]);
+        unsigned long long w[8];
+        cic_weights(d[k], d[k], d[k], w);
+        mass[k] = 0;
+        for (int c = 0; c < 8; c++) mass[k] += w[c];
+    }
+}
+
 }  // extern "C"

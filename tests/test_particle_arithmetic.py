@@ -54,3 +54,24 @@ def test_deposit_cells_stay_in_the_grid(host, N, L, dtype):
     for site in (0, N // 2, N - 1):
         check(N, ctypes.c_double(L), ctypes.c_long(x.size), site, _p(x), _p(base))
         assert base.min() >= -N and base.max() < 2 * N
+
+
+# cells of 1.5 and 2.5, whose reciprocals round, and of 2; positions everywhere and
+# a few floats around every cell edge
+@pytest.mark.parametrize("N,L", [(256, 384.0), (96, 240.0), (256, 512.0)])
+def test_float_cell_offsets_and_mass(host, N, L):
+    rng = np.random.default_rng(N)
+    edge = np.float32(np.arange(N) * (L / N))
+    near = [edge]
+    for to in (-np.inf, np.inf):
+        x = edge
+        for _ in range(4):
+            x = np.nextafter(x, np.float32(to))
+            near.append(x)
+    x = np.concatenate([rng.random(1000000) * L, *near]).astype(np.float32)
+    d = np.empty_like(x)
+    mass = np.empty(x.size, np.uint64)
+    host.check_cell_mass(N, ctypes.c_double(L), ctypes.c_long(x.size), _p(x), _p(d), _p(mass))
+    assert d.min() >= 0 and d.max() <= 1
+    # eight weights, each from four roundings of 2^-24 of itself and one to a unit
+    assert np.abs(mass.astype(np.int64) - (1 << 24)).max() <= 8
