@@ -49,7 +49,7 @@ __device__ __forceinline__ float fwrap_float(float x, float Lf, double L) {
 // one axis of the TSC window (src/grids_interp.c:291-296): the three taps with
 // non-zero weight, in the reference's loop order.  X is in cell units.
 template <typename M>
-__device__ __forceinline__ void tsc_axis(M X, int& i0, M w[3]) {
+__host__ __device__ __forceinline__ void tsc_axis(M X, int& i0, M w[3]) {
 #pragma clang fp contract(off)
     const int iX = (int)floor(X);
     const M d = X - iX;
@@ -65,19 +65,18 @@ __device__ __forceinline__ void tsc_axis(M X, int& i0, M w[3]) {
 
 // tsc_axis in half the instructions, the same bits.  The reference forms xx =
 // |X - tap| and picks its formula by xx < 1/2 and xx < 3/2.  With u = X - (nearest
-// tap), exact in floating point, the taps lie at 1 + u, |u| and 1 - u (the
-// reference's xx, each rounded once as there), and the formulas are known: where
-// two meet, at xx = 1/2, they agree.  A cell past the int range, an infinity or a
-// NaN has all weights zero, as there.  For the kernels that read their taps from
-// memory; k_displace_tile_ref, held to 128 registers, is slower with it (512^3:
-// 24.3 -> 25.3 ms for the realization).
-__device__ __forceinline__ void tsc_axis_short(double X, int& i0, double w[3]) {
+// tap), which is exact (X - floor(X) is not, for X in (-1/2, 0)), the taps lie at
+// 1 + u, |u| and 1 - u (the reference's xx, each rounded once as there), and the
+// formulas are known: where two meet, at xx = 1/2, they agree.  A cell past the int
+// range, an infinity or a NaN has all weights zero, as there.  For the kernels that
+// read their taps from memory; k_displace_tile_ref, held to 128 registers, is slower
+// with it (512^3: 24.3 -> 25.3 ms for the realization).
+__host__ __device__ __forceinline__ void tsc_axis_short(double X, int& i0, double w[3]) {
 #pragma clang fp contract(off)
     const int iX = (int)floor(X);
     const double d = X - iX;
-    const bool low = d < 0.5;  // reference loops from floor(d-1.5)
-    i0 = low ? iX - 1 : iX;
-    const double u = low ? d : d - 1;
+    i0 = d < 0.5 ? iX - 1 : iX;  // reference loops from floor(d-1.5)
+    const double u = X - ((double)i0 + 1);
     const bool ok = fabs(u) <= 0.5;
     const double l = 1.5 - (1 + u), r = 1.5 - (1 - u);
     w[0] = ok ? 0.5 * l * l : 0;

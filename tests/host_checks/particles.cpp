@@ -48,4 +48,12 @@ void check_cell_mass(int N, double L, long n, const float* x, float* d,
     }
 }
 
+// TSC cells and weights: the reference's formulas and the kernels' short form
+void check_tsc_axis(long n, const double* x, int* i, double* w) {
+    for (long k = 0; k < n; k++) tsc_axis(x[k], i[k], w + 3 * k);
+}
+void check_tsc_axis_short(long n, const double* x, int* i, double* w) {
+    for (long k = 0; k < n; k++) tsc_axis_short(x[k], i[k], w + 3 * k);
+}
+
 }  // extern "C"

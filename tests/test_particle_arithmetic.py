@@ -75,3 +75,26 @@ def test_float_cell_offsets_and_mass(host, N, L):
     assert d.min() >= 0 and d.max() <= 1
     # eight weights, each from four roundings of 2^-24 of itself and one to a unit
     assert np.abs(mass.astype(np.int64) - (1 << 24)).max() <= 8
+
+
+# moved coordinates are not wrapped yet: below zero, where X - floor(X) rounds, and
+# on both sides of cell edges and half cells
+def test_tsc_weights_have_the_reference_bits(host):
+    rng = np.random.default_rng(1)
+    marks = np.arange(-40, 41) / 2.0
+    near = [marks]
+    for to in (-np.inf, np.inf):
+        x = marks
+        for _ in range(3):
+            x = np.nextafter(x, to)
+            near.append(x)
+    x = np.concatenate([rng.uniform(a, b, 300000) for a, b in ((-0.5, 0), (-5, 5), (0, 300))] +
+                       [-10.0 ** rng.uniform(-300, 0, 100000), *near, [1e15, -1e15, np.inf, np.nan]])
+    res = []
+    for check in (host.check_tsc_axis, host.check_tsc_axis_short):
+        i, w = np.empty(x.size, np.int32), np.empty((x.size, 3))
+        check(ctypes.c_long(x.size), _p(x), _p(i), _p(w))
+        res.append((i, w))
+    assert np.array_equal(res[0][1].view(np.uint64), res[1][1].view(np.uint64))
+    inside = np.abs(x) < 1e9
+    assert np.array_equal(res[0][0][inside], res[1][0][inside])
