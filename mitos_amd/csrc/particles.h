@@ -128,53 +128,56 @@ __device__ __forceinline__ TscTaps<O> tsc_taps(double X, int N, float invN, O st
     return t;
 }
 
-// the sums of G grids at one position.  FLAT: the z taps of all the wave's lanes
-// are consecutive (no lane wraps), so a row is one 16-byte and one 8-byte load;
-// that pays with velocities (250^3 particles on 256^3, moves and velocities: 3.20
-// -> 2.54 ms) and not for moves alone (512^3: 7.76 -> 8.30 ms).
-template <int G, bool FLAT, typename O>
-__device__ __forceinline__ void tsc_sums(const double* const* box, const TscTaps<O>& x,
-                                         const TscTaps<O>& y, const TscTaps<O>& z, double* sum) {
+// the sum of a grid at one position, all 27 values loaded before the first is used
+// (left free, the compiler waits for each row of three).  FLAT: the z taps are
+// consecutive in memory, so a row is one 16-byte and one 8-byte load.
+template <bool FLAT, typename O>
+__device__ __forceinline__ double tsc_sum(const double* box, const TscTaps<O>& x,
+                                          const TscTaps<O>& y, const TscTaps<O>& z) {
 #pragma clang fp contract(off)
     typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
+    const char* p = reinterpret_cast<const char*>(box);
+    double v[9][3];
 #pragma unroll
-    for (int g = 0; g < G; g++) sum[g] = 0;
+    for (int r = 0; r < 9; r++) {
+        const O row = x.o[r / 3] + y.o[r % 3];
+        if constexpr (FLAT) {
+            const pair q = *reinterpret_cast<const pair*>(p + (O)(row + z.o[0]));
+            v[r][0] = q.x;
+            v[r][1] = q.y;
+            v[r][2] = *reinterpret_cast<const double*>(p + (O)(row + z.o[0] + 16));
+        } else {
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-#pragma unroll
-        for (int b = 0; b < 3; b++) {
-            const O row = x.o[a] + y.o[b];
-            const double wab = x.w[a] * y.w[b];
-            const double w0 = wab * z.w[0], w1 = wab * z.w[1], w2 = wab * z.w[2];
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-                const char* p = reinterpret_cast<const char*>(box[g]);
-                double v0, v1, v2;
-                if constexpr (FLAT) {
-                    const pair v = *reinterpret_cast<const pair*>(p + (O)(row + z.o[0]));
-                    v0 = v.x;
-                    v1 = v.y;
-                    v2 = *reinterpret_cast<const double*>(p + (O)(row + z.o[0] + 16));
-                } else {
-                    v0 = *reinterpret_cast<const double*>(p + (O)(row + z.o[0]));
-                    v1 = *reinterpret_cast<const double*>(p + (O)(row + z.o[1]));
-                    v2 = *reinterpret_cast<const double*>(p + (O)(row + z.o[2]));
-                }
-                sum[g] += v0 * w0;
-                sum[g] += v1 * w1;
-                sum[g] += v2 * w2;
-            }
+            for (int c = 0; c < 3; c++)
+                v[r][c] = *reinterpret_cast<const double*>(p + (O)(row + z.o[c]));
         }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    double sum = 0;
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        const double wab = x.w[r / 3] * y.w[r % 3];
+        sum += v[r][0] * (wab * z.w[0]);
+        sum += v[r][1] * (wab * z.w[1]);
+        sum += v[r][2] * (wab * z.w[2]);
+    }
+    return sum;
 }
-template <int G, bool FLAT, typename O>
-__device__ __forceinline__ void tsc_gather(const double* const* box, const TscTaps<O>& x,
-                                           const TscTaps<O>& y, const TscTaps<O>& z,
-                                           double* sum) {
-    if (FLAT && __ballot(z.o[2] != z.o[0] + 16) == 0)
-        tsc_sums<G, true>(box, x, y, z, sum);
-    else
-        tsc_sums<G, false>(box, x, y, z, sum);
+// TEST: flat rows for a wave none of whose lanes wraps in z and most of whose
+// neighbouring lanes lie within eight cells in z.  Lanes in scattered places meet a
+// line each, and the wide loads are the slower ones (moves of 256^3 particles on
+// 256^3 with one kind of load: lattice order flat 0.92 ms, single values 1.05 ms;
+// random order 10.7 and 9.3 ms).
+template <bool TEST, typename O>
+__device__ __forceinline__ double tsc_gather(const double* box, const TscTaps<O>& x,
+                                             const TscTaps<O>& y, const TscTaps<O>& z) {
+    if constexpr (TEST) {
+        const int dz = (int)(z.o[0] - __shfl_xor(z.o[0], 1, 64));
+        if (__popcll(__ballot(dz >= -64 && dz <= 64)) >= 40 &&
+            __ballot(z.o[2] != z.o[0] + 16) == 0)
+            return tsc_sum<true>(box, x, y, z);
+    }
+    return tsc_sum<false>(box, x, y, z);
 }
 
 // src/particle.c:87-129: lattice position of particle p (index x*M*M+y*M+z)
@@ -202,107 +205,109 @@ __global__ void k_lattice(int M, float spacing, long long first_id, float* X, fl
     if (ids) ids[p] = p + first_id;
 }
 
-// Order in which the particle kernels of the drop-in calls walk their arrays.
-// Particles written by mitos_lattice lie in lattice order, where 256 neighbours
-// in memory are a thin line along z; the taps of a compact block share far more
-// lines.  So an array of M^3 particles is walked in blocks of 8 x 8 x 16 of its
-// lattice indices (any other length in memory order).  This is an order of work
-// only: each particle's result is its own.
-struct ParticleOrder {
-    long long n;
-    int M;  // 0: memory order
-    unsigned nty, ntz, blocks;
-};
-inline ParticleOrder particle_order(long long n) {
-    ParticleOrder o{n, 0, 0, 0, (unsigned)((n + 1023) / 1024)};
-    long long M = (long long)llround(cbrt((double)n));
-    if (M >= 16 && M * M * M == n) {
-        o.M = (int)M;
-        o.nty = (unsigned)((M + 7) / 8);
-        o.ntz = (unsigned)((M + 15) / 16);
-        o.blocks = (unsigned)((M + 7) / 8) * o.nty * o.ntz;
-    }
-    return o;
-}
-// particle k (0..3) of a thread of 256, or -1
-__device__ __forceinline__ long long ordered_particle(const ParticleOrder& o, unsigned block,
-                                                      int k) {
-    if (o.M == 0) {
-        const long long p = (long long)block * 1024 + k * 256 + threadIdx.x;
-        return p < o.n ? p : -1;
-    }
-    const int z = (int)(block % o.ntz) * 16 + (int)(threadIdx.x & 15);
-    const int y = (int)(block / o.ntz % o.nty) * 8 + (int)((threadIdx.x >> 4) & 7);
-    const int x = (int)(block / (o.ntz * o.nty)) * 8 + (int)(threadIdx.x >> 7) + 2 * k;
-    if (x >= o.M || y >= o.M || z >= o.M) return -1;
-    return ((long long)x * o.M + y) * o.M + z;
-}
-
 // The particle loop of src/mitos.c:824-908 and :1072-1077 over padded grids (rows
 // of N + 2): the three sequential moves (DISP), velocities by TSC at the moved,
 // not yet wrapped positions, stored as float (VEL), and the wrap, in the
 // reference's double arithmetic.  A move changes one coordinate, so one axis is
-// formed anew per gather; the three velocities share their taps.  Bound by the L1
-// cache's line accesses (33 per load, 0.83 per cycle and CU: neighbours' taps lie
-// in different rows once they moved) and, at half the time, by the FP64 sums.
-// Against one particle per thread in memory order: 512^3 moves 11.5 -> 7.8 ms,
-// 250^3 moves and velocities on 256^3 4.0 -> 2.5 ms.  Staging the taps' box of
-// 1024 particles in LDS measured 9.4 and 3.6 ms (80 KB windows leave two
-// work-groups per CU to hide the loads of each stage).
+// formed anew per gather.
+// Particles written by mitos_lattice lie in lattice order, where 256 neighbours in
+// memory are a thin line along z; the taps of a compact block share far more lines.
+// M > 0: the array holds M^3 particles and a work-group takes a block of 4 x 8 x 8
+// of its lattice indices; M = 0: any length, in memory order.  This is an order of
+// work only: each particle's result is its own.
+// Bound by the L1 cache's line accesses (neighbours' taps lie in different rows once
+// they moved) and, at half the time, by the FP64 sums.  One particle a thread:
+// several in turn leave small arrays too few waves (4096 particles on 256^3: 95
+// against 27 us) and scattered ones too few loads in flight.  Three velocities summed
+// together share their taps' weights but thrash L1 (512^3 at moved positions 11.9 ms,
+// one grid after the other 8.9 ms).  With 27 loads in flight a thread, two waves a
+// SIMD after moves and three without lose least to evictions from L1 (moves of 512^3
+// at two, three, four waves: lattice order 6.7, 6.1, 5.9 ms, random order 92, 98, 103
+// ms).  Staging the taps' box of 1024 particles in LDS measured slower (80 KB windows
+// leave two work-groups per CU to hide the loads of each stage).
 struct DisplaceGrids {
     const double* psi[3];
     const double* vel[3];
 };
-template <bool DISP, bool VEL, typename O>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-    k_displace_grids(DisplaceGrids g, int N, double boxlen, ParticleOrder order, float* X,
-                     float* Y, float* Z, float* VX, float* VY, float* VZ) {
+constexpr int kDisplaceX = 4, kDisplaceY = 8, kDisplaceZ = 8;
+template <bool DISP, bool VEL, bool BLOCKS, typename O>
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(DISP ? 2 : 3, DISP ? 2 : 3)))
+    k_displace_grids(DisplaceGrids g, int N, double boxlen, long long n, int M, unsigned block0,
+                     float* X, float* Y, float* Z, float* VX, float* VY, float* VZ) {
 #pragma clang fp contract(off)
-    const unsigned block = xcd_block(blockIdx.x, gridDim.x);
+    const unsigned block = block0 + xcd_block(blockIdx.x, gridDim.x);
+    long long p;
+    if constexpr (BLOCKS) {
+        const unsigned ntz = (unsigned)(M + kDisplaceZ - 1) / kDisplaceZ,
+                       nty = (unsigned)(M + kDisplaceY - 1) / kDisplaceY;
+        const int qz = (int)(block % ntz) * kDisplaceZ + (int)(threadIdx.x % kDisplaceZ);
+        const int qy = (int)(block / ntz % nty) * kDisplaceY +
+                       (int)(threadIdx.x / kDisplaceZ % kDisplaceY);
+        const int qx = (int)(block / (ntz * nty)) * kDisplaceX +
+                       (int)(threadIdx.x / (kDisplaceZ * kDisplaceY));
+        if (qx >= M || qy >= M || qz >= M) return;
+        p = ((long long)qx * M + qy) * M + qz;
+    } else {
+        p = (long long)block * 256 + threadIdx.x;
+        if (p >= n) return;
+    }
+    constexpr bool TEST = BLOCKS || VEL;
     const float invN = 1.0f / N;
     const O sz = 8, sy = (O)(N + 2) * 8, sx = sy * (O)N;
-#pragma unroll 1
-    for (int k = 0; k < 4; k++) {
-        const long long p = ordered_particle(order, block, k);
-        if (p < 0) continue;
-        float x = X[p], y = Y[p], z = Z[p];
-        TscTaps<O> tx = tsc_taps<O>((double)x * N / boxlen, N, invN, sx);
-        TscTaps<O> ty = tsc_taps<O>((double)y * N / boxlen, N, invN, sy);
-        TscTaps<O> tz = tsc_taps<O>((double)z * N / boxlen, N, invN, sz);
-        double d[3];
-        if constexpr (DISP) {
-            tsc_gather<1, VEL>(&g.psi[0], tx, ty, tz, d);
-            x = (float)((double)x - d[0]);
-            tx = tsc_taps<O>((double)x * N / boxlen, N, invN, sx);
-            tsc_gather<1, VEL>(&g.psi[1], tx, ty, tz, d);
-            y = (float)((double)y - d[0]);
-            ty = tsc_taps<O>((double)y * N / boxlen, N, invN, sy);
-            tsc_gather<1, VEL>(&g.psi[2], tx, ty, tz, d);
-            z = (float)((double)z - d[0]);
-        }
-        if constexpr (VEL) {
-            if constexpr (DISP) tz = tsc_taps<O>((double)z * N / boxlen, N, invN, sz);
-            tsc_gather<3, VEL>(g.vel, tx, ty, tz, d);
-            VX[p] = (float)d[0];
-            VY[p] = (float)d[1];
-            VZ[p] = (float)d[2];
-        }
-        X[p] = (float)fwrap_fast(x, boxlen);
-        Y[p] = (float)fwrap_fast(y, boxlen);
-        Z[p] = (float)fwrap_fast(z, boxlen);
+    float x = X[p], y = Y[p], z = Z[p];
+    TscTaps<O> tx = tsc_taps<O>((double)x * N / boxlen, N, invN, sx);
+    TscTaps<O> ty = tsc_taps<O>((double)y * N / boxlen, N, invN, sy);
+    TscTaps<O> tz = tsc_taps<O>((double)z * N / boxlen, N, invN, sz);
+    if constexpr (DISP) {
+        x = (float)((double)x - tsc_gather<TEST>(g.psi[0], tx, ty, tz));
+        tx = tsc_taps<O>((double)x * N / boxlen, N, invN, sx);
+        y = (float)((double)y - tsc_gather<TEST>(g.psi[1], tx, ty, tz));
+        ty = tsc_taps<O>((double)y * N / boxlen, N, invN, sy);
+        z = (float)((double)z - tsc_gather<TEST>(g.psi[2], tx, ty, tz));
     }
+    if constexpr (VEL) {
+        if constexpr (DISP) tz = tsc_taps<O>((double)z * N / boxlen, N, invN, sz);
+        VX[p] = (float)tsc_gather<TEST>(g.vel[0], tx, ty, tz);
+        VY[p] = (float)tsc_gather<TEST>(g.vel[1], tx, ty, tz);
+        VZ[p] = (float)tsc_gather<TEST>(g.vel[2], tx, ty, tz);
+    }
+    X[p] = (float)fwrap_fast(x, boxlen);
+    Y[p] = (float)fwrap_fast(y, boxlen);
+    Z[p] = (float)fwrap_fast(z, boxlen);
 }
+// Blocks for M^3 particles from M = 64 on: below, and for other lengths, the array is
+// walked in memory order (the cut blocks of 50^3 cost as much as they save).  Against
+// one particle a thread in memory order with all axes formed anew per gather (moves,
+// moves and velocities, velocities alone):
+//   512^3 on 512^3, lattice order  9.6 -> 6.7, 31.2 -> 13.1, 9.8 -> 5.1 ms
+//   512^3 on 512^3, random order   92.5 -> 92.4, 199 -> 186, 99.7 -> 97.2 ms
+//   250^3 on 256^3, cells of 0.6   1.74 -> 0.94, 5.72 -> 2.25, 1.15 -> 0.65 ms
+//   the same and one more (memory order)  1.74 -> 1.61, 5.71 -> 4.10, 1.15 -> 0.64 ms
+//   200^3 on 64^3, random order    2.13 -> 1.80, 5.42 -> 3.51, 2.53 -> 1.67 ms
+//   16^3 on 64^3                   20 -> 19, 28 -> 24, 20 -> 17 us
 template <bool DISP, bool VEL>
 inline void displace_grids_launch(const DisplaceGrids& g, int N, double boxlen, long long npart,
                                   float* X, float* Y, float* Z, float* VX, float* VY, float* VZ,
                                   hipStream_t s) {
-    const ParticleOrder order = particle_order(npart);
-    if ((unsigned long long)(N + 2) * N * N * 8 < (1ull << 32))
-        hipLaunchKernelGGL((k_displace_grids<DISP, VEL, unsigned>), dim3(order.blocks), dim3(256),
-                           0, s, g, N, boxlen, order, X, Y, Z, VX, VY, VZ);
-    else
-        hipLaunchKernelGGL((k_displace_grids<DISP, VEL, unsigned long long>), dim3(order.blocks),
-                           dim3(256), 0, s, g, N, boxlen, order, X, Y, Z, VX, VY, VZ);
+    const long long M = (long long)llround(cbrt((double)npart));
+    const bool in_blocks = M >= 64 && M * M * M == npart;
+    const bool narrow = (unsigned long long)(N + 2) * N * N * 8 < (1ull << 32);
+    const long long blocks = in_blocks ? (M + kDisplaceX - 1) / kDisplaceX *
+                                             ((M + kDisplaceY - 1) / kDisplaceY) *
+                                             ((M + kDisplaceZ - 1) / kDisplaceZ)
+                                       : (npart + 255) / 256;
+    const auto kern =
+        in_blocks ? (narrow ? k_displace_grids<DISP, VEL, true, unsigned>
+                            : k_displace_grids<DISP, VEL, true, unsigned long long>)
+                  : (narrow ? k_displace_grids<DISP, VEL, false, unsigned>
+                            : k_displace_grids<DISP, VEL, false, unsigned long long>);
+    // a launch holds fewer than 2^32 threads
+    const long long cap = 1 << 23;
+    for (long long b = 0; b < blocks; b += cap)
+        hipLaunchKernelGGL(kern, dim3((unsigned)(blocks - b < cap ? blocks - b : cap)), dim3(256),
+                           0, s, g, N, boxlen, npart, (int)(in_blocks ? M : 0), (unsigned)b, X, Y,
+                           Z, VX, VY, VZ);
 }
 
 // ---- displacement grids with a periodic z halo -------------------------------------
