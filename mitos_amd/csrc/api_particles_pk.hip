@@ -275,7 +275,7 @@ extern "C" int mitos_cic_overdensity(int N, double boxlen, long long npart, cons
     // sorted by tile when that pays and its buffers can be had, else one atomic
     // per corner of every particle: the same integers
     const size_t sort_bytes = cic_sort_bytes(N, npart);
-    void* sort_ws = cic_sort_pays(N, npart) ? workspace(8, sort_bytes) : nullptr;
+    void* sort_ws = cic_sort_pays(N, npart, sort_bytes) ? workspace(8, sort_bytes) : nullptr;
     if (!sort_ws) (void)hipGetLastError();  // no room for the sort: the atomics need none
     if (sort_ws)
         MITOS_TRY(set_last_error(

@@ -44,14 +44,30 @@ int cic_sorted(const float* X, const float* Y, const float* Z, long long npart, 
                double boxlen, unsigned long long* grid, void* ws, size_t ws_bytes,
                hipStream_t s);
 
-// Whether the sort is the faster deposit.  Its five launches and the visit to
-// every tile cost about 60 us; the atomics take about 0.36 us per thousand
-// particles in random order and half of that in lattice order.  Measured on a
-// 64^3 grid, sorted against atomics: 262144 particles 72 against 46 us (lattice
-// order) and 66 against 111 us (random), 10^6 particles 101 against 214 and 94
-// against 364 us.
-inline bool cic_sort_pays(int N, long long npart) {
-    return N <= 4096 && npart >= 524288 && npart >= (long long)cic_sort_dims(N).ntiles;
+// Whether the sort is the faster deposit with a workspace of ws_bytes.  A pass of up
+// to its capacity is four launches (40 to 60 us on small grids), and every tile that
+// holds particles clears and flushes its window (about 8 ns of the whole deposit); the
+// atomics take about 0.36 us per thousand particles in random order, 0.07 to 0.2 in
+// lattice order and more on grids below 64^3.  So a pass holds 524288 particles or
+// more, the deposit 200 a tile, the figure at which lattice order breaks even (random
+// order at about 30; the order is not known here).  mitos_cic_overdensity, atomics
+// against sorted, lattice order / random:
+//    64^3, 600000           134,   76 / 231,   72 us     (9375 a tile)
+//   256^3, 600000           160,  177 / 290,  186 us     (146)
+//   256^3, 1000000          195,  186 / 424,  219 us     (244)
+//   512^3, 4000000         1130, 1243 / 2087, 1299 us    (122)
+//   512^3, 16000000        2115, 1914 / 6479, 2423 us    (488)
+//  1024^3, 600000          4655, 5550 / 4692, 6296 us    (2)
+//  1024^3, 30000000        8977, 9640 / 16253, 10245 us  (114)
+// and the FP32 realization of 128^3 particles on 16^3, where the displacement grids
+// hold 4890 particles a pass: 2.6, 16.4 ms.
+inline bool cic_sort_pays(int N, long long npart, size_t ws_bytes) {
+    if (N > 4096 || ws_bytes < cic_sort_tables(N)) return false;
+    const long long tiles = cic_sort_dims(N).ntiles;
+    const long long room = (long long)((ws_bytes - cic_sort_tables(N)) / kCicSortParticle);
+    const long long most = room < kCicSortPass ? room : kCicSortPass;
+    const long long pass = npart < most ? npart : most;
+    return pass >= 524288 && pass >= 32 * tiles && npart >= 200 * tiles;
 }
 
 }  // namespace mitos

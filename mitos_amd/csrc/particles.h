@@ -35,14 +35,14 @@ __host__ __device__ __forceinline__ double fwrap_fast(double x, double L) {
     return r;
 }
 
-__device__ __noinline__ inline float fwrap_float_far(float x, double L) {
+__host__ __device__ __noinline__ inline float fwrap_float_far(float x, double L) {
     return (float)fwrap_fast(x, L);
 }
 
 // Float periodic wrap of a float position: x itself on [0, Lf), Lf = (float)L
 // (positions written by the displacement kernels lie there), the double wrap
 // otherwise.
-__device__ __forceinline__ float fwrap_float(float x, float Lf, double L) {
+__host__ __device__ __forceinline__ float fwrap_float(float x, float Lf, double L) {
     return (x >= 0.0f && x < Lf) ? x : fwrap_float_far(x, L);
 }
 
@@ -1177,8 +1177,9 @@ __global__ void __launch_bounds__(TXN / PP * TY * TZ) __attribute__((amdgpu_wave
 // (000, 100, 010, 001, 110, 101, 011, 111).
 // (P: float, the particle arrays; double, the positions of the FP64 adjoint)
 template <typename P>
-__device__ __forceinline__ void cic_cell(P X, P Y, P Z, int N, double boxlen, int& iX, int& iY,
-                                         int& iZ, double& dx, double& dy, double& dz) {
+__host__ __device__ __forceinline__ void cic_cell(P X, P Y, P Z, int N, double boxlen, int& iX,
+                                                  int& iY, int& iZ, double& dx, double& dy,
+                                                  double& dz) {
 #pragma clang fp contract(off)
     const double cell = boxlen / N;
     const double Xc = fwrap_fast((double)X, boxlen) / cell;
@@ -1211,9 +1212,9 @@ __host__ __device__ __forceinline__ void cic_weights(double dx, double dy, doubl
 // cell is formed as X - iX * cell with one rounding, so it keeps the float
 // position's accuracy; weights in units of 2^-24 (the float mantissa), so a
 // 32-bit cell holds the mass of 256 particles.
-__device__ __forceinline__ void cic_cell_f(float X, float Y, float Z, int N, float cell,
-                                           float cinv, double boxlen, int& iX, int& iY, int& iZ,
-                                           float& dx, float& dy, float& dz) {
+__host__ __device__ __forceinline__ void cic_cell_f(float X, float Y, float Z, int N, float cell,
+                                                    float cinv, double boxlen, int& iX, int& iY,
+                                                    int& iZ, float& dx, float& dy, float& dz) {
     const float Lf = (float)boxlen;
     const float P[3] = {fwrap_float(X, Lf, boxlen), fwrap_float(Y, Lf, boxlen),
                         fwrap_float(Z, Lf, boxlen)};

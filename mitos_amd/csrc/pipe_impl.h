@@ -427,9 +427,9 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
                 }
                 // another lattice than the grid's: sorted by tile, in the A grids
                 // (free once the displacement grids are made)
-                if (cic_sort_pays(NN, nl))
-                    return cic_sorted<M>(X, Y, Z, nl, NN, L, cic(), A,
-                                         sizeof(cx<T>) * (size_t)csize * 3, s);
+                const size_t room = sizeof(cx<T>) * (size_t)csize * 3;
+                if (cic_sort_pays(NN, nl, room))
+                    return cic_sorted<M>(X, Y, Z, nl, NN, L, cic(), A, room, s);
                 hipLaunchKernelGGL(k_cic<M>, dim3(nblk(nl)), dim3(256), 0, s, X, Y, Z, nl, NN, L,
                                    cic());
                 return launch_status();

@@ -1,4 +1,5 @@
 import os
+import subprocess
 import sys
 
 import pytest
@@ -28,3 +29,16 @@ def gpu():
     import mitos_amd.ic as ic
     ic.lib()
     return ic
+
+
+@pytest.fixture(scope="session")
+def host_checks(tmp_path_factory):
+    """The arithmetic of the particle kernels compiled for the host (ctypes)."""
+    import ctypes
+    out = str(tmp_path_factory.mktemp("host_checks") / "particles.so")
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "-x", "hip",
+                    "--offload-host-only", "-std=c++20", "-O1", "-fPIC", "-ffp-contract=off",
+                    "-shared", "-o", out,
+                    os.path.join(ROOT, "tests", "host_checks", "particles.cpp")],
+                   check=True, capture_output=True)
+    return ctypes.CDLL(out)

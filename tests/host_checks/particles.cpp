@@ -6,7 +6,42 @@
 
 using namespace mitos;
 
+namespace {
+
+template <typename W>
+void deposit(int N, double L, long n, const float* X, const float* Y, const float* Z,
+             unsigned long long* grid) {
+    for (long k = 0; k < n; k++) {
+        int i[3];
+        W d[3];
+        if constexpr (sizeof(W) == 8)
+            cic_cell(X[k], Y[k], Z[k], N, L, i[0], i[1], i[2], d[0], d[1], d[2]);
+        else
+            cic_cell_f(X[k], Y[k], Z[k], N, (float)(L / N), (float)(N / L), L, i[0], i[1], i[2],
+                       d[0], d[1], d[2]);
+        unsigned long long w[8];
+        cic_weights(d[0], d[1], d[2], w);
+        const int corner[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1},
+                                  {1, 1, 0}, {1, 0, 1}, {0, 1, 1}, {1, 1, 1}};
+        for (int c = 0; c < 8; c++)
+            grid[((size_t)wrapi(i[0] + corner[c][0], N) * N + wrapi(i[1] + corner[c][1], N)) * N +
+                 wrapi(i[2] + corner[c][2], N)] += w[c];
+    }
+}
+
+}  // namespace
+
 extern "C" {
+
+// the fixed-point CIC sums of particles in any order, one after the other
+void check_deposit_f(int N, double L, long n, const float* X, const float* Y, const float* Z,
+                     unsigned long long* grid) {
+    deposit<float>(N, L, n, X, Y, Z, grid);
+}
+void check_deposit_d(int N, double L, long n, const float* X, const float* Y, const float* Z,
+                     unsigned long long* grid) {
+    deposit<double>(N, L, n, X, Y, Z, grid);
+}
 
 void check_wrapf(int N, long n, const int* i, int* out) {
     for (long k = 0; k < n; k++) out[k] = wrapf(i[k], N, 1.0f / N);

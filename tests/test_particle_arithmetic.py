@@ -1,24 +1,9 @@
 """The index and weight arithmetic of the particle kernels, compiled for the host:
 positions far from the box, at the edges of cells and of the box."""
 import ctypes
-import os
-import subprocess
 
 import numpy as np
 import pytest
-
-HERE = os.path.dirname(os.path.abspath(__file__))
-
-
-@pytest.fixture(scope="module")
-def host(tmp_path_factory):
-    out = str(tmp_path_factory.mktemp("host_checks") / "particles.so")
-    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-std=c++20", "-O1", "-fPIC",
-                    "-ffp-contract=off", "-shared", "-o", out,
-                    os.path.join(HERE, "host_checks", "particles.cpp")],
-                   check=True, capture_output=True)
-    return ctypes.CDLL(out)
 
 
 def _p(a):
@@ -27,14 +12,14 @@ def _p(a):
 
 # every compiled grid size: powers of two, whose reciprocal is exact, and 3 * 2^k
 @pytest.mark.parametrize("N", [8, 16, 24, 48, 96, 256, 384, 1024, 1536])
-def test_wrapped_cells_stay_in_the_grid(host, N):
+def test_wrapped_cells_stay_in_the_grid(host_checks, N):
     rng = np.random.default_rng(N)
     near = rng.integers(-(1 << 22) + 1, 1 << 22, 200000)
     far = rng.integers(-(1 << 31), 1 << 31, 200000)
     ends = np.array([0, -1, N, N - 1, -N, -(1 << 31), (1 << 31) - 1])
     i = np.concatenate([near, far, ends]).astype(np.int32)
     out = np.empty_like(i)
-    host.check_wrapf(N, ctypes.c_long(i.size), _p(i), _p(out))
+    host_checks.check_wrapf(N, ctypes.c_long(i.size), _p(i), _p(out))
     assert out.min() >= 0 and out.max() < N
     assert np.array_equal(out[:near.size], np.mod(near, N))
 
@@ -43,14 +28,14 @@ def test_wrapped_cells_stay_in_the_grid(host, N):
 # more box lengths than a float resolves, infinities and NaN
 @pytest.mark.parametrize("N,L", [(32, 48.0), (96, 1000 / 3), (256, 500.0), (256, 512.0)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-def test_deposit_cells_stay_in_the_grid(host, N, L, dtype):
+def test_deposit_cells_stay_in_the_grid(host_checks, N, L, dtype):
     rng = np.random.default_rng(N)
     scale = 10.0 ** rng.uniform(0, 30, 200000)
     x = np.concatenate([L * scale * rng.choice([-1, 1], scale.size), L * rng.random(200000),
                         [0, L, np.nextafter(dtype(L), dtype(0)), -1e-30, np.inf, -np.inf, np.nan]])
     x = x.astype(dtype)
     base = np.empty(x.size, np.int32)
-    check = host.check_lattice_cell_f if dtype == np.float32 else host.check_lattice_cell_d
+    check = host_checks.check_lattice_cell_f if dtype == np.float32 else host_checks.check_lattice_cell_d
     for site in (0, N // 2, N - 1):
         check(N, ctypes.c_double(L), ctypes.c_long(x.size), site, _p(x), _p(base))
         assert base.min() >= -N and base.max() < 2 * N
@@ -59,7 +44,7 @@ def test_deposit_cells_stay_in_the_grid(host, N, L, dtype):
 # cells of 1.5 and 2.5, whose reciprocals round, and of 2; positions everywhere and
 # a few floats around every cell edge
 @pytest.mark.parametrize("N,L", [(256, 384.0), (96, 240.0), (256, 512.0)])
-def test_float_cell_offsets_and_mass(host, N, L):
+def test_float_cell_offsets_and_mass(host_checks, N, L):
     rng = np.random.default_rng(N)
     edge = np.float32(np.arange(N) * (L / N))
     near = [edge]
@@ -71,7 +56,7 @@ def test_float_cell_offsets_and_mass(host, N, L):
     x = np.concatenate([rng.random(1000000) * L, *near]).astype(np.float32)
     d = np.empty_like(x)
     mass = np.empty(x.size, np.uint64)
-    host.check_cell_mass(N, ctypes.c_double(L), ctypes.c_long(x.size), _p(x), _p(d), _p(mass))
+    host_checks.check_cell_mass(N, ctypes.c_double(L), ctypes.c_long(x.size), _p(x), _p(d), _p(mass))
     assert d.min() >= 0 and d.max() <= 1
     # eight weights, each from four roundings of 2^-24 of itself and one to a unit
     assert np.abs(mass.astype(np.int64) - (1 << 24)).max() <= 8
@@ -79,7 +64,7 @@ def test_float_cell_offsets_and_mass(host, N, L):
 
 # moved coordinates are not wrapped yet: below zero, where X - floor(X) rounds, and
 # on both sides of cell edges and half cells
-def test_tsc_weights_have_the_reference_bits(host):
+def test_tsc_weights_have_the_reference_bits(host_checks):
     rng = np.random.default_rng(1)
     marks = np.arange(-40, 41) / 2.0
     near = [marks]
@@ -91,7 +76,7 @@ def test_tsc_weights_have_the_reference_bits(host):
     x = np.concatenate([rng.uniform(a, b, 300000) for a, b in ((-0.5, 0), (-5, 5), (0, 300))] +
                        [-10.0 ** rng.uniform(-300, 0, 100000), *near, [1e15, -1e15, np.inf, np.nan]])
     res = []
-    for check in (host.check_tsc_axis, host.check_tsc_axis_short):
+    for check in (host_checks.check_tsc_axis, host_checks.check_tsc_axis_short):
         i, w = np.empty(x.size, np.int32), np.empty((x.size, 3))
         check(ctypes.c_long(x.size), _p(x), _p(i), _p(w))
         res.append((i, w))
