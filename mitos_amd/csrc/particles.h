@@ -410,18 +410,19 @@ __device__ __forceinline__ M tsc_halo(const T* __restrict__ box, unsigned rs, in
 // src/mitos.c:827-863 then :1072-1077 for the particles of an Ml^3 lattice
 // (src/particle.c:87-129, spacing (float)L / Ml) over halo-padded
 // displacement grids of N^3 cells.  Work-groups of 256 threads over blocks of
-// 8 x 8 x 16 sites (x, y, z), four x planes' sites a thread; the FP64 instance
+// `planes` x 8 x 16 sites (x, y, z), two planes' sites at a time; the FP64 instance
 // (M = double) keeps the reference's arithmetic, the FP32 one (M = float) moves
 // particles in float.  81 taps a particle in 27 loads of 12 bytes: a block's taps
 // lie in a few KB of L1, a lattice row's spread over nine rows of the grid that the
 // next row's work-group fetches again (350^3 particles on 384^3 in FP32: a row of
-// 256 sites per work-group 3.53 ms, blocks 2.12 ms; bound by L1 accesses).
+// 256 sites per work-group 3.53 ms, blocks of eight planes 2.12 ms; bound by L1
+// accesses).
 template <typename T, typename M>
 __global__ void __launch_bounds__(256)
     k_displace_lattice(const T* __restrict__ px, const T* __restrict__ py,
-                       const T* __restrict__ pz, unsigned rs, int N, int Ml, double boxlen,
-                       float spacing, float* __restrict__ X, float* __restrict__ Y,
-                       float* __restrict__ Z) {
+                       const T* __restrict__ pz, unsigned rs, int N, int Ml, int planes,
+                       double boxlen, float spacing, float* __restrict__ X,
+                       float* __restrict__ Y, float* __restrict__ Z) {
 #pragma clang fp contract(off)
     constexpr bool REF = sizeof(M) == 8;
     const unsigned block = xcd_block(blockIdx.x, gridDim.x);
@@ -429,12 +430,12 @@ __global__ void __launch_bounds__(256)
     const unsigned br = block / ntz;
     const int qz = (int)(block - br * ntz) * 16 + (int)(threadIdx.x & 15);
     const int qy = (int)(br % nty) * 8 + (int)((threadIdx.x >> 4) & 7);
-    const int qx0 = (int)(br / nty) * 8 + (int)(threadIdx.x >> 7);
+    const int qx0 = (int)(br / nty) * planes, qx1 = min(Ml, qx0 + planes);
     if (qy >= Ml || qz >= Ml) return;
     const float invN = 1.0f / N;
     const double bl = boxlen;
 #pragma unroll 1
-    for (int qx = qx0; qx < min(Ml, qx0 + 8); qx += 2) {
+    for (int qx = qx0 + (int)(threadIdx.x >> 7); qx < qx1; qx += 2) {
         float x = qx * spacing, y = qy * spacing, z = qz * spacing;  // src/particle.c:107-109
         // cell coordinates as the reference forms them (double x*N/boxlen);
         // weights, sums and moves in M
@@ -453,8 +454,12 @@ __global__ void __launch_bounds__(256)
         Z[p] = (float)fwrap_fast(z, boxlen);
     }
 }
+// x planes of a block: below 64^3 sites two, one site a thread, or few waves run (8^3 in
+// FP64 19.7 -> 12 us)
+inline int displace_lattice_planes(int Ml) { return Ml < 64 ? 2 : 8; }
 inline unsigned displace_lattice_blocks(int Ml) {
-    return (unsigned)((long)((Ml + 7) / 8) * ((Ml + 7) / 8) * ((Ml + 15) / 16));
+    const int planes = displace_lattice_planes(Ml);
+    return (unsigned)((long)((Ml + planes - 1) / planes) * ((Ml + 7) / 8) * ((Ml + 15) / 16));
 }
 
 // FP32 lattice displacement.  For a coordinate on the lattice the TSC window

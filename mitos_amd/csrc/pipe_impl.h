@@ -360,7 +360,8 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
                     // at each particle's position
                     hipLaunchKernelGGL((k_displace_lattice<T, M>),
                                        dim3(displace_lattice_blocks(Ml)), dim3(256), 0, s,
-                                       psi(0), psi(1), psi(2), rs, NN, Ml, L, spacing, X, Y, Z);
+                                       psi(0), psi(1), psi(2), rs, NN, Ml,
+                                       displace_lattice_planes(Ml), L, spacing, X, Y, Z);
                 } else if (STENCIL && NN % 16 == 0 && tsc_tile) {
                     auto tile = [&](auto kern, int txn, int ty, int tz, int pp) {
                         const dim3 gridt(
@@ -406,7 +407,8 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
                 } else {
                     hipLaunchKernelGGL((k_displace_lattice<T, M>),
                                        dim3(displace_lattice_blocks(NN)), dim3(256), 0, s,
-                                       psi(0), psi(1), psi(2), rs, NN, NN, L, spacing, X, Y, Z);
+                                       psi(0), psi(1), psi(2), rs, NN, NN,
+                                       displace_lattice_planes(NN), L, spacing, X, Y, Z);
                 }
                 return launch_status();
             }));
