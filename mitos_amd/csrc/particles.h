@@ -1407,7 +1407,7 @@ __global__ void __launch_bounds__(256)
 }
 
 // The adjoint's moves and deposit on grids without deposit tiles (N not a
-// multiple of 32): positions kept in T for the deposit (their float copies go
+// multiple of 32) and at 32^3: positions kept in T for the deposit (their float copies go
 // to X/Y/Z), fixed-point weights 2^-shift with global atomics (order
 // independent).
 template <typename T>

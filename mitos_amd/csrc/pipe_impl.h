@@ -321,9 +321,10 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
             // differentiates, positions in T up to the deposit.  FP64 positions lie
             // in the A grids (free once the displacement grids are made).
             MITOS_TRY(timed(s, "move_deposit", 3 * Rg + 12.0 * np + 8.0 * np, [&] {
-                if constexpr (NN % 32 == 0) {
+                if constexpr (NN % 32 == 0 && NN > 32) {
                     // moves, then the tiled LDS deposit of the pipeline: 0.06 ms at
                     // 96^3 in FP64, a global atomic per corner and particle 0.30 ms
+                    // (at 32^3 one launch is the faster: 164 against 175 us the forward)
                     T* xt = reinterpret_cast<T*>(a(0));
                     T* yt = reinterpret_cast<T*>(a(1));
                     T* zt = reinterpret_cast<T*>(a(2));

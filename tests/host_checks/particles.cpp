@@ -9,6 +9,17 @@ using namespace mitos;
 namespace {
 
 template <typename W>
+void add_cloud(int N, const int i[3], const W d[3], unsigned long long* grid) {
+    unsigned long long w[8];
+    cic_weights(d[0], d[1], d[2], w);
+    const int corner[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1},
+                              {1, 1, 0}, {1, 0, 1}, {0, 1, 1}, {1, 1, 1}};
+    for (int c = 0; c < 8; c++)
+        grid[((size_t)wrapi(i[0] + corner[c][0], N) * N + wrapi(i[1] + corner[c][1], N)) * N +
+             wrapi(i[2] + corner[c][2], N)] += w[c];
+}
+
+template <typename W>
 void deposit(int N, double L, long n, const float* X, const float* Y, const float* Z,
              unsigned long long* grid) {
     for (long k = 0; k < n; k++) {
@@ -19,13 +30,7 @@ void deposit(int N, double L, long n, const float* X, const float* Y, const floa
         else
             cic_cell_f(X[k], Y[k], Z[k], N, (float)(L / N), (float)(N / L), L, i[0], i[1], i[2],
                        d[0], d[1], d[2]);
-        unsigned long long w[8];
-        cic_weights(d[0], d[1], d[2], w);
-        const int corner[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1},
-                                  {1, 1, 0}, {1, 0, 1}, {0, 1, 1}, {1, 1, 1}};
-        for (int c = 0; c < 8; c++)
-            grid[((size_t)wrapi(i[0] + corner[c][0], N) * N + wrapi(i[1] + corner[c][1], N)) * N +
-                 wrapi(i[2] + corner[c][2], N)] += w[c];
+        add_cloud(N, i, d, grid);
     }
 }
 
@@ -66,6 +71,19 @@ void check_lattice_cell_d(int N, double L, long n, int site, const double* x, in
         cic_lattice_cell<double, true>(p, p, p, N, L, 0.0f, 0.0f, site, site, site, rx, ry, rz,
                                        fx, fy, fz);
         base[k] = site + rx;
+    }
+}
+
+// the same with the cells of the FP32 adjoint
+void check_deposit_t(int N, double L, long n, const float* X, const float* Y, const float* Z,
+                     unsigned long long* grid) {
+    for (long k = 0; k < n; k++) {
+        int i[3];
+        float d[3];
+        cic_cell_t(X[k], (float)(N / L), N, i[0], d[0]);
+        cic_cell_t(Y[k], (float)(N / L), N, i[1], d[1]);
+        cic_cell_t(Z[k], (float)(N / L), N, i[2], d[2]);
+        add_cloud(N, i, d, grid);
     }
 }
 
