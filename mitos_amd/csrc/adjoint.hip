@@ -487,7 +487,7 @@ static int backward(Pipe<T>* P, const mitos_ic_config& cfg, const cx<T>* noise,
         hipLaunchKernelGGL((k_adj_pk<T>), dim3(nblk(nh)), dim3(256), 0, s, P->K, hs, N, edges,
                            pk_bin_cinv(N, cfg.bins), cfg.bins, dcoef, sfwd, w2);
         MITOS_TRY(launch_status());
-        MITOS_TRY((c2r_3d<T>(N, P->K, hs, P->a(0), P->a(1), grho, (long)N, (T)1, OpNone(), s)));
+        MITOS_TRY((c2r_3d<T>(N, P->K, hs, P->a(0), P->a(1), hs, grho, (long)N, (T)1, OpNone(), s)));
         MITOS_HIP_CHECK(hipStreamSynchronize(s));  // dcoef is host-backed until here
     } else {
         hipLaunchKernelGGL((k_fill<T>), dim3(nblk(n3)), dim3(256), 0, s, grho, n3, (T)0);
@@ -529,7 +529,7 @@ static int backward(Pipe<T>* P, const mitos_ic_config& cfg, const cx<T>* noise,
     T* A3[3] = {Ax, Ay, Az};
     for (int a = 0; a < 3; a++) {
         RealRowLoader<T> ld{A3[a], (long)N, 0};
-        MITOS_TRY((r2c_3d<T>(N, ld, P->K, P->a(0), R[a], hs, OpNone(), s)));
+        MITOS_TRY((r2c_3d<T>(N, ld, P->K, P->a(0), hs, R[a], hs, OpNone(), s)));
     }
     // 4. combine adjoint -> G1 (a1), GD (K)
     const double* win = window_table(N, L, 3);
@@ -543,7 +543,7 @@ static int backward(Pipe<T>* P, const mitos_ic_config& cfg, const cx<T>* noise,
     if (cfg.run2lpt) {
         // 5. dL/ddelta2(x)
         T* gd2 = reinterpret_cast<T*>(P->b(0));
-        MITOS_TRY((c2r_3d<T>(N, P->K, hs, P->a(0), P->a(2), gd2, (long)N, (T)1, OpNone(), s)));
+        MITOS_TRY((c2r_3d<T>(N, P->K, hs, P->a(0), P->a(2), hs, gd2, (long)N, (T)1, OpNone(), s)));
         // 6. recompute phi1(k) and the six phi_,ij
         const double A = amplitude_cached(cfg.n_s, cfg.gamma, cfg.sigma8);
         const double* amp = phi1_table(N, L, A, cfg.n_s, cfg.gamma);
@@ -556,7 +556,7 @@ static int backward(Pipe<T>* P, const mitos_ic_config& cfg, const cx<T>* noise,
                     reinterpret_cast<T*>(P->b(3)), reinterpret_cast<T*>(P->b(4)),
                     reinterpret_cast<T*>(P->b(5)), reinterpret_cast<T*>(P->a(2))};
         for (int q = 0; q < 6; q++)
-            MITOS_TRY((c2r_3d<T>(N, P->K, hs, P->a(0), P->a(0), ph[q], (long)N,
+            MITOS_TRY((c2r_3d<T>(N, P->K, hs, P->a(0), P->a(0), hs, ph[q], (long)N,
                                  (T)(1.0 / boxvol), OpHess{N, q, dk}, s)));
         // 7. Hessian-minor adjoint, then back to k-space into G1
         hipLaunchKernelGGL((k_adj_minors<T>), dim3(nblk(n3)), dim3(256), 0, s, ph[0], ph[1],
@@ -564,7 +564,7 @@ static int backward(Pipe<T>* P, const mitos_ic_config& cfg, const cx<T>* noise,
         MITOS_TRY(launch_status());
         for (int q = 0; q < 6; q++) {
             RealRowLoader<T> ld{ph[q], (long)N, 0};
-            MITOS_TRY((r2c_3d<T>(N, ld, P->K, P->a(0), P->K, hs, OpNone(), s)));
+            MITOS_TRY((r2c_3d<T>(N, ld, P->K, P->a(0), hs, P->K, hs, OpNone(), s)));
             hipLaunchKernelGGL((k_adj_hess_acc<T>), dim3(nblk(nh)), dim3(256), 0, s, G1, P->K, hs,
                                N, q, dk, boxvol);
             MITOS_TRY(launch_status());

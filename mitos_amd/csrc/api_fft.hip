@@ -237,29 +237,35 @@ int scale_complex(cx<T>* a, long n, double s) {
     return api_sync();
 }
 
-// Two work grids of the transforms, or one used twice where two do not fit
+// Work grids of a transform and their row stride: whole lines, dense rows where only
+// those fit.  Two up to 32 MB each (128^3), else one used twice (see c2r_3d).
 template <typename T>
-bool work_grids(int N, cx<T>** w1, cx<T>** w2) {
-    const size_t bytes = work_grid_bytes<T>(N);
-    if ((*w1 = (cx<T>*)workspace(0, 2 * bytes))) {
-        *w2 = *w1 + bytes / sizeof(cx<T>);
+bool work_grids(int N, cx<T>** w1, cx<T>** w2, long* hs) {
+    const size_t bytes = work_grid_bytes<T>(N), second = bytes <= (32u << 20) ? bytes : 0;
+    *hs = work_row<T>(N);
+    *w1 = (cx<T>*)workspace(0, bytes + second);
+    if (*w1) {
+        *w2 = *w1 + second / sizeof(cx<T>);
         return true;
     }
     (void)hipGetLastError();
-    *w2 = *w1 = (cx<T>*)workspace(0, bytes);
+    *hs = N / 2 + 1;
+    *w1 = *w2 = (cx<T>*)workspace(0, sizeof(cx<T>) * half_elems(N));
+    if (!*w1) (void)hipGetLastError();
     return *w1 != nullptr;
 }
 
 // r2c of an N^3 array with row stride rs into the (N, N, N/2+1) layout, times
-// scale, issued on the library stream
+// scale, issued on the library stream; in place in the output where no work grid fits
 template <typename T, typename OPX>
 int r2c_issue(int N, const T* in, long rs, cx<T>* out, OPX ox) {
     if (!in || !out) return MITOS_ERR_ARG;
     if (!size_supported(N)) return MITOS_ERR_UNSUPPORTED;
     cx<T>*w1, *w2;
-    if (!work_grids(N, &w1, &w2)) return MITOS_ERR_ALLOC;
+    long hs;
+    if (!work_grids(N, &w1, &w2, &hs)) w1 = w2 = out;
     RealRowLoader<T> ld{in, rs, 0};
-    return r2c_3d<T>(N, ld, w1, w2, out, N / 2 + 1, ox, api_stream());
+    return r2c_3d<T>(N, ld, w1, w2, hs, out, N / 2 + 1, ox, api_stream());
 }
 
 template <typename T>
@@ -267,8 +273,9 @@ int c2r_issue(int N, const cx<T>* in, T* out, long rs, double scale) {
     if (!in || !out) return MITOS_ERR_ARG;
     if (!size_supported(N)) return MITOS_ERR_UNSUPPORTED;
     cx<T>*w1, *w2;
-    if (!work_grids(N, &w1, &w2)) return MITOS_ERR_ALLOC;
-    return c2r_3d<T>(N, in, N / 2 + 1, w1, w2, out, rs, (T)scale, OpNone(), api_stream());
+    long hs;
+    if (!work_grids(N, &w1, &w2, &hs)) return MITOS_ERR_ALLOC;
+    return c2r_3d<T>(N, in, N / 2 + 1, w1, w2, hs, out, rs, (T)scale, OpNone(), api_stream());
 }
 
 // unnormalised r2c of an N^3 array with row stride rs into the (N, N, N/2+1) layout

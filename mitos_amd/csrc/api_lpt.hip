@@ -7,11 +7,11 @@
 // (multi_launch.h), so each line is read once per axis; c2r of the potential
 // itself is the z pass of one of the six.  The six grids between the y and z
 // passes exist as slabs of x planes, halves (2LPT) or quarters (Monge-Ampere,
-// which also holds six real slabs): with the transforms' work grids nine grids
-// in all, as the separate transforms held.  Smaller slabs, which the
+// which also holds six real slabs): with the transforms' work grid eight grids
+// in all, nine were held by the separate transforms.  Smaller slabs, which the
 // memory-side cache would hold, are slower (2LPT at 384^3: halves 6.2 ms, slabs
 // of 128 MB 8.2 ms): the launches get too short.
-// solve2LPT at 256^3: 3.46 -> 1.8 ms, bound by HBM and the memory-side cache
+// solve2LPT at 256^3: 3.46 -> 1.60 ms, bound by HBM and the memory-side cache
 // (6.6 GB in its passes).
 #include <string.h>
 

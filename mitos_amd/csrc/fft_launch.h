@@ -324,17 +324,19 @@ int zr2c_pass_tuned(int variant, LOADER loader, cx<T>* out, long hs, int nbatch,
 }
 
 // ---- composed 3D transforms ---------------------------------------------------
-// The passes between the caller's arrays run through two work grids w1, w2 of
-// whole 128-byte rows (work_row elements), out of place: a pass over the dense
-// rows of N/2+1 values splits every tile row over two lines, and one in place
-// streams slower.  The pass at the caller's dense grid is the y pass, whose tiles
-// of one plane meet in L2 (512^3 FP64: 0.44 ms reading and 0.49 ms writing it, an
-// x pass 0.54 and 0.64 ms).  Whole transforms at 512^3 in FP64, against in-place
-// passes over dense rows: c2r 1.58 -> 1.31 ms, r2c 1.61 -> 1.36 ms, bound by HBM
-// (three passes of 2.15 GB at 4.8 TB/s).  w2 == w1 transforms in place.  Schedules: variant 0 of the strided passes, variant 1 of
-// the z passes, which measured within 3% of the fastest at every size but FP64
-// 768^3 r2c (the 16 values per thread of variant 0 take twice as long in FP64 at
-// 256^3 and 512^3: r2c 907 against 424 us).
+// The passes between the caller's arrays run through work grids w1, w2 of rows of
+// whs, whole 128-byte lines (work_row elements) where there is room: a pass over the
+// dense rows of N/2+1 values splits every tile row over two lines.  w2 == w1 passes
+// x in place, which the drop-in calls do above 128^3: a second grid gains 4 to 11% at
+// 128^3 and 5% of an r2c at 512^3 (1.40 against 1.48 ms in FP64), but loses 21% at
+// 256^3 (206 against 163 us), where the arrays then leave the memory-side cache.  The
+// pass at the caller's dense grid is the y pass, whose tiles of one plane meet in L2
+// (512^3 FP64: 0.44 ms reading and 0.49 ms writing it, an x pass 0.54 and 0.64 ms).
+// Whole transforms in FP64 against passes over dense rows: 512^3 c2r 1.55 -> 1.31 ms,
+// r2c 1.57 -> 1.48 ms; 256^3 211 -> 164 us, 199 -> 164 us; bound by HBM (512^3: three
+// passes of 2.15 GB at 4.8 TB/s).  Schedules: variant 0 of the strided passes, variant
+// 1 of the z passes (the 16 values per thread of variant 0 take twice as long in FP64
+// at 256^3 and 512^3: z r2c 907 against 424 us).
 template <typename T>
 inline long work_row(int N) {
     const long q = 128 / (long)sizeof(cx<T>);
@@ -348,25 +350,23 @@ inline size_t work_grid_bytes(int N) {
 // c2r: y (in -> w1, values through op.pre), x (w1 -> w2), z (w2 -> out).  The
 // input is left unchanged (unless it is w1).
 template <typename T, typename OP>
-int c2r_3d(int N, const cx<T>* in, long ihs, cx<T>* w1, cx<T>* w2, T* out, long rs, T scale,
-           OP op, hipStream_t s) {
-    const long hs = work_row<T>(N);
+int c2r_3d(int N, const cx<T>* in, long ihs, cx<T>* w1, cx<T>* w2, long whs, T* out, long rs,
+           T scale, OP op, hipStream_t s) {
     return with_size(N, [&]<int NN>() -> int {
-        MITOS_TRY((strided_pass_v<T, NN, 1, 1, 0>(in, ihs, w1, hs, op, s)));
-        MITOS_TRY((strided_pass_v<T, NN, 0, 1, 0>(w1, hs, w2, hs, OpNone(), s)));
-        return zc2r_pass_v<T, NN, 1, 0>(w2, out, hs, rs, 1, 0, 0, scale, OpNone(), s);
+        MITOS_TRY((strided_pass_v<T, NN, 1, 1, 0>(in, ihs, w1, whs, op, s)));
+        MITOS_TRY((strided_pass_v<T, NN, 0, 1, 0>(w1, whs, w2, whs, OpNone(), s)));
+        return zc2r_pass_v<T, NN, 1, 0>(w2, out, whs, rs, 1, 0, 0, scale, OpNone(), s);
     });
 }
 
 // r2c: z (loader -> w1), x (w1 -> w2), y (w2 -> out, values through op.post).
 template <typename T, typename LOADER, typename OP>
-int r2c_3d(int N, LOADER loader, cx<T>* w1, cx<T>* w2, cx<T>* out, long ohs, OP op,
+int r2c_3d(int N, LOADER loader, cx<T>* w1, cx<T>* w2, long whs, cx<T>* out, long ohs, OP op,
            hipStream_t s) {
-    const long hs = work_row<T>(N);
     return with_size(N, [&]<int NN>() -> int {
-        MITOS_TRY((zr2c_pass_v<T, NN, 1>(loader, w1, hs, 1, 0, OpNone(), s)));
-        MITOS_TRY((strided_pass_v<T, NN, 0, -1, 0>(w1, hs, w2, hs, OpNone(), s)));
-        return strided_pass_v<T, NN, 1, -1, 0>(w2, hs, out, ohs, op, s);
+        MITOS_TRY((zr2c_pass_v<T, NN, 1>(loader, w1, whs, 1, 0, OpNone(), s)));
+        MITOS_TRY((strided_pass_v<T, NN, 0, -1, 0>(w1, whs, w2, whs, OpNone(), s)));
+        return strided_pass_v<T, NN, 1, -1, 0>(w2, whs, out, ohs, op, s);
     });
 }
 

@@ -297,8 +297,8 @@ static int unstencil_psi(Pipe<T>* P, int N, T* out, hipStream_t s) {
     const int masks[3] = {7, 6, 4};
     for (int i = 0; i < 3; i++) {
         RealRowLoader<T> ld{P->psi(i) + MITOS_PSI_SO, P->prs(), 0};
-        MITOS_TRY((r2c_3d<T>(N, ld, P->a(0), P->a(1), P->K, P->hs, OpNone(), s)));
-        MITOS_TRY((c2r_3d<T>(N, P->K, P->hs, P->a(0), P->a(1), out + (size_t)i * N * N * N,
+        MITOS_TRY((r2c_3d<T>(N, ld, P->a(0), P->a(1), P->hs, P->K, P->hs, OpNone(), s)));
+        MITOS_TRY((c2r_3d<T>(N, P->K, P->hs, P->a(0), P->a(1), P->hs, out + (size_t)i * N * N * N,
                              (long)N, (T)1, OpUnstencil{S, masks[i], norm}, s)));
     }
     return MITOS_OK;
