@@ -95,8 +95,12 @@ int launch_apply(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double box
                  const KSpec& ks, const double* tab, const TransferTab& t = TransferTab{}) {
     const long n = nx * N * (N / 2 + 1);
     if (n <= 0) return api_sync();
-    hipLaunchKernelGGL((k_apply_kernel<TW, TR, HOW>), dim3(nblk(n, kApplyBlock)), dim3(256), 0,
-                       api_stream(), w, (long)(N / 2 + 1), r, N, x0, nx, boxlen, ks, tab, t);
+    const bool small = n < kApplySmall;
+    const auto kern = small ? k_apply_kernel<TW, TR, HOW, 1>
+                            : k_apply_kernel<TW, TR, HOW, kApplyModes>;
+    const int modes = small ? 256 : 256 * kApplyModes;
+    hipLaunchKernelGGL(kern, dim3(nblk(n, modes)), dim3(256), 0, api_stream(), w,
+                       (long)(N / 2 + 1), r, N, x0, nx, boxlen, ks, tab, t);
     MITOS_TRY(launch_status());
     return api_sync();
 }
@@ -208,23 +212,30 @@ int apply_kernel(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double box
     if (kr == MITOS_ERR_UNSUPPORTED)
         return apply_kernel_host<TW, TR>(w, r, N, x0, nx, boxlen, compute, params);
     MITOS_TRY(kr);
-    // tables of a window's N factors, and of the spectra's powers and logarithms
-    // over n^2 from 64^3 on, where the grid has 21 modes and more per entry
-    if (ks.id == KID_UNDO_WINDOW) {
-        double* tab = (double*)workspace(9, sizeof(double) * N);
-        if (!tab) return MITOS_ERR_ALLOC;
-        hipLaunchKernelGGL(k_window_factors, dim3(nblk(N)), dim3(256), 0, api_stream(), ks, N,
-                           boxlen, tab);
-        return launch_apply<APPLY_WINDOW>(w, r, N, x0, nx, boxlen, ks, tab);
+    // Tables of a window's N factors, and of the spectra's powers and logarithms over
+    // n^2: a launch more, so where there are enough modes, for the spectra also enough
+    // per entry (a slab has few).  Direct against table, call and wait: window 64^3 (2^17
+    // modes) 19.6, 19.8 us, 128^3 (2^20) 38, 24 us; power law 64^3 18.5, 20.8 us, 128^3
+    // 30, 25 us; of 1024^3 in FP32 four planes (2.7 modes an entry) power law 39, 42 us,
+    // BBKS 70, 54 us, sixteen planes 100, 77 us and 220, 89 us.  Where no scratch can be
+    // had they are evaluated directly as well.
+    const long n = nx * N * (N / 2 + 1), n2 = 3L * (N / 2) * (N / 2) + 1;
+    if (ks.id == KID_UNDO_WINDOW && n >= (1L << 18)) {
+        if (double* tab = (double*)workspace(9, sizeof(double) * N)) {
+            hipLaunchKernelGGL(k_window_factors, dim3(nblk(N)), dim3(256), 0, api_stream(), ks,
+                               N, boxlen, tab);
+            return launch_apply<APPLY_WINDOW>(w, r, N, x0, nx, boxlen, ks, tab);
+        }
+        (void)hipGetLastError();
     }
-    if (N >= 64 && (ks.id == KID_POWER_NO_TRANSFER || ks.id == KID_SQRT_POWER_LAW ||
-                    ks.id == KID_BBKS)) {
-        const long n2 = 3L * (N / 2) * (N / 2) + 1;
-        double* tab = (double*)workspace(9, sizeof(double) * n2);
-        if (!tab) return MITOS_ERR_ALLOC;
-        hipLaunchKernelGGL(k_radial_values, dim3(nblk(n2)), dim3(256), 0, api_stream(), ks, n2,
-                           boxlen, tab);
-        return launch_apply<APPLY_RADIAL>(w, r, N, x0, nx, boxlen, ks, tab);
+    if ((ks.id == KID_POWER_NO_TRANSFER || ks.id == KID_SQRT_POWER_LAW || ks.id == KID_BBKS) &&
+        n >= (1L << 19) && n >= (ks.id == KID_BBKS ? 2 : 8) * n2) {
+        if (double* tab = (double*)workspace(9, sizeof(double) * n2)) {
+            hipLaunchKernelGGL(k_radial_values, dim3(nblk(n2)), dim3(256), 0, api_stream(), ks,
+                               n2, boxlen, tab);
+            return launch_apply<APPLY_RADIAL>(w, r, N, x0, nx, boxlen, ks, tab);
+        }
+        (void)hipGetLastError();
     }
     return launch_apply<APPLY_DIRECT>(w, r, N, x0, nx, boxlen, ks, nullptr);
 }
@@ -529,8 +540,8 @@ int apply_padded_issue(cx<double>* w, long whs, const struct distributed_grid* d
                        const KSpec& ks) {
     const int N = dg->N;
     const long n = (long)N * N * (N / 2 + 1);
-    hipLaunchKernelGGL((k_apply_kernel<double, double, APPLY_DIRECT>), dim3(nblk(n, kApplyBlock)),
-                       dim3(256), 0, api_stream(), w, whs,
+    hipLaunchKernelGGL((k_apply_kernel<double, double, APPLY_DIRECT, kApplyModes>),
+                       dim3(nblk(n, 256 * kApplyModes)), dim3(256), 0, api_stream(), w, whs,
                        reinterpret_cast<const cx<double>*>(dg->fbox), N, 0L, (long)N, dg->boxlen,
                        ks, (const double*)nullptr, TransferTab{});
     return launch_status();

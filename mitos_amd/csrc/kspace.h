@@ -126,14 +126,17 @@ __host__ __device__ __forceinline__ double transfer_value(const TransferTab& t, 
 }
 
 // ---- write = read * kernel over the half grid (src/fft.c:257-302) ----------------
-// A work-group takes 1024 consecutive modes of the dense grid, so every access
+// A work-group takes 1024 (K = 4) consecutive modes of the dense grid, so every access
 // is whole lines whatever the row length; it divides its first index once, and
 // a mode's row and z' follow from small offsets.  Bound by HBM: read and write
 // once.  Against one mode per thread with 64-bit divisions, and sin and pow per
 // mode: the TSC window and a derivative at 384^3 in FP64 0.68 -> 0.31 ms (5.9
 // TB/s), the CIC window at 512^3 in FP32 1.19 -> 0.28 ms; a spectrum at 512^3 in
 // FP64 1.6 -> 0.75 ms, bound by the scattered reads of its table.
-constexpr int kApplyBlock = 1024;
+// Below 2^21 modes a thread takes one (K = 1), as four leave too few waves (a
+// derivative, call and wait: 32^3 17.5 -> 16.6 us, 128^3 22.6 -> 22.1 us).
+constexpr int kApplyModes = 4;
+constexpr long kApplySmall = 1L << 21;
 
 // small / d for 0 <= small < 2^20, d >= 2
 __device__ __forceinline__ int small_div(int small, int d, float inv) {
@@ -145,12 +148,11 @@ __device__ __forceinline__ int small_div(int small, int d, float inv) {
 // The block's modes of nx x-slabs from x0: load(id) of all of a thread's first
 // (dense offsets; a store to w may alias a later load of r), then f(id, value,
 // x, y, z).
-template <typename V, typename LOAD, typename F>
+template <int K, typename V, typename LOAD, typename F>
 __device__ __forceinline__ void for_block_modes(int N, long x0, long nx, LOAD&& load, F&& f) {
-    constexpr int K = kApplyBlock / 256;
     const int H = N / 2 + 1;
     const long n = nx * N * H;
-    const long e0 = (long)blockIdx.x * kApplyBlock;
+    const long e0 = (long)blockIdx.x * (256 * K);
     V v[K];
 #pragma unroll
     for (int j = 0; j < K; j++) {
@@ -185,14 +187,14 @@ enum { APPLY_DIRECT = 0, APPLY_WINDOW = 1, APPLY_RADIAL = 2, APPLY_TRANSFER = 3 
 
 // TW/TR may be float (the _float variants compute the product in double, as C
 // does for fftwf_complex * double complex).  r is dense, w has rows of whs.
-template <typename TW, typename TR, int HOW>
+template <typename TW, typename TR, int HOW, int K>
 __global__ void __launch_bounds__(256)
     k_apply_kernel(cx<TW>* w, long whs, const cx<TR>* r, int N, long x0, long nx, double boxlen,
                    KSpec ks, const double* __restrict__ tab, TransferTab t) {
 #pragma clang fp contract(off)
     const double dk = 2 * M_PI / boxlen;
     auto load = [&](long id) { return ld(r + id); };
-    for_block_modes<cx<TR>>(N, x0, nx, load, [&](long id, cx<TR> a, int x, int y, int z) {
+    for_block_modes<K, cx<TR>>(N, x0, nx, load, [&](long id, cx<TR> a, int x, int y, int z) {
         cx<double> kv;
         if constexpr (HOW == APPLY_DIRECT) {
             double kx, ky, kz, k;
