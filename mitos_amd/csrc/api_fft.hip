@@ -94,7 +94,7 @@ template <int HOW, typename TW, typename TR>
 int launch_apply(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double boxlen,
                  const KSpec& ks, const double* tab, const TransferTab& t = TransferTab{}) {
     const long n = nx * N * (N / 2 + 1);
-    if (n <= 0) return api_sync();
+    if (n <= 0) return MITOS_ERR_DEVICE;  // as a launch of no work-groups fails
     const bool small = n < kApplySmall;
     const auto kern = small ? k_apply_kernel<TW, TR, HOW, 1>
                             : k_apply_kernel<TW, TR, HOW, kApplyModes>;

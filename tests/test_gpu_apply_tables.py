@@ -54,3 +54,17 @@ def test_tables_and_formulas_agree(gpu, N, x0, nx, name):
             got[0, 0, 0] = want[0, 0, 0] = 0
     # one rounding to float of a product in double
     assert torch.all((got - want).abs() <= 2.0 ** -23 * want.abs() + 1e-30)
+
+
+@pytest.mark.parametrize("name,kw", [("kernel_dx", {}),
+                                     ("kernel_undo_Hermite_window", dict(order=2, N=16, boxlen=9.0)),
+                                     ("kernel_bbks_transfer", dict(Gamma=0.2))])
+def test_empty_slab_is_refused(gpu, name, kw):
+    import torch
+    print("case empty slab", name, flush=True)
+    f = torch.zeros(1, 16, 9, dtype=torch.complex64, device="cuda")
+    torch.cuda.synchronize()
+    p = gpu.kernel_params(name, **kw) if kw else None
+    assert gpu.lib().fft_apply_kernel_float_mpi(
+        f.data_ptr(), f.data_ptr(), 16, 0, 0, 9.0, gpu.kernel_ptr(name),
+        ctypes.cast(ctypes.byref(p), ctypes.c_void_p) if p is not None else None) == 3
