@@ -91,7 +91,7 @@ int kspec_from_callback(void (*compute)(struct kernel*), const void* params, int
 }
 
 template <int HOW, typename TW, typename TR>
-int launch_apply(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double boxlen,
+int issue_apply(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double boxlen,
                  const KSpec& ks, const double* tab, const TransferTab& t = TransferTab{}) {
     const long n = nx * N * (N / 2 + 1);
     if (n <= 0) return MITOS_ERR_DEVICE;  // as a launch of no work-groups fails
@@ -101,8 +101,7 @@ int launch_apply(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double box
     const int modes = small ? 256 : 256 * kApplyModes;
     hipLaunchKernelGGL(kern, dim3(nblk(n, modes)), dim3(256), 0, api_stream(), w,
                        (long)(N / 2 + 1), r, N, x0, nx, boxlen, ks, tab, t);
-    MITOS_TRY(launch_status());
-    return api_sync();
+    return launch_status();
 }
 
 // kernel_(inv_)transfer_function: the k vector and the selected function's
@@ -122,7 +121,8 @@ int apply_transfer(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double b
     MITOS_HIP_CHECK(copy_sync(d, pt->k, sizeof(double) * ks, hipMemcpyHostToDevice));
     MITOS_HIP_CHECK(copy_sync(d + ks, rows, sizeof(double) * 2 * ks, hipMemcpyHostToDevice));
     TransferTab t{d, d + ks, d + 2 * ks, ks, sp->u_tau, invert};
-    return launch_apply<APPLY_TRANSFER>(w, r, N, x0, nx, boxlen, KSpec{}, nullptr, t);
+    MITOS_TRY((issue_apply<APPLY_TRANSFER>(w, r, N, x0, nx, boxlen, KSpec{}, nullptr, t)));
+    return api_sync();
 }
 
 // Any other callback: evaluated on the host for every mode with the
@@ -199,6 +199,37 @@ int apply_kernel_host(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, doubl
     return rc;
 }
 
+// a kernel with a device form, issued on the library stream
+template <typename TW, typename TR>
+int device_apply(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double boxlen,
+                 const KSpec& ks) {
+    // Tables of a window's N factors, and of the spectra's powers and logarithms over
+    // n^2: a launch more, so where there are enough modes, for the spectra also enough
+    // per entry (a slab has few).  Direct against table, call and wait: window 64^3 (2^17
+    // modes) 19.6, 19.8 us, 128^3 (2^20) 38, 24 us; power law 64^3 18.5, 20.8 us, 128^3
+    // 30, 25 us; of 1024^3 in FP32 four planes (2.7 modes an entry) power law 39, 42 us,
+    // BBKS 70, 54 us, sixteen planes 100, 77 us and 220, 89 us.  Where no scratch can be
+    // had they are evaluated directly as well.
+    ScratchLock hold;
+    const long n = nx * N * (N / 2 + 1), n2 = 3L * (N / 2) * (N / 2) + 1;
+    if (ks.id == KID_UNDO_WINDOW && n >= (1L << 18)) {
+        if (double* tab = (double*)workspace(SLOT_APPLY_TABLE, sizeof(double) * N)) {
+            hipLaunchKernelGGL(k_window_factors, dim3(nblk(N)), dim3(256), 0, api_stream(), ks,
+                               N, boxlen, tab);
+            return issue_apply<APPLY_WINDOW>(w, r, N, x0, nx, boxlen, ks, tab);
+        }
+    }
+    if ((ks.id == KID_POWER_NO_TRANSFER || ks.id == KID_SQRT_POWER_LAW || ks.id == KID_BBKS) &&
+        n >= (1L << 19) && n >= (ks.id == KID_BBKS ? 2 : 8) * n2) {
+        if (double* tab = (double*)workspace(SLOT_APPLY_TABLE, sizeof(double) * n2)) {
+            hipLaunchKernelGGL(k_radial_values, dim3(nblk(n2)), dim3(256), 0, api_stream(), ks,
+                               n2, boxlen, tab);
+            return issue_apply<APPLY_RADIAL>(w, r, N, x0, nx, boxlen, ks, tab);
+        }
+    }
+    return issue_apply<APPLY_DIRECT>(w, r, N, x0, nx, boxlen, ks, nullptr);
+}
+
 template <typename TW, typename TR>
 int apply_kernel(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double boxlen,
                  void (*compute)(struct kernel*), const void* params) {
@@ -212,32 +243,8 @@ int apply_kernel(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double box
     if (kr == MITOS_ERR_UNSUPPORTED)
         return apply_kernel_host<TW, TR>(w, r, N, x0, nx, boxlen, compute, params);
     MITOS_TRY(kr);
-    // Tables of a window's N factors, and of the spectra's powers and logarithms over
-    // n^2: a launch more, so where there are enough modes, for the spectra also enough
-    // per entry (a slab has few).  Direct against table, call and wait: window 64^3 (2^17
-    // modes) 19.6, 19.8 us, 128^3 (2^20) 38, 24 us; power law 64^3 18.5, 20.8 us, 128^3
-    // 30, 25 us; of 1024^3 in FP32 four planes (2.7 modes an entry) power law 39, 42 us,
-    // BBKS 70, 54 us, sixteen planes 100, 77 us and 220, 89 us.  Where no scratch can be
-    // had they are evaluated directly as well.
-    const long n = nx * N * (N / 2 + 1), n2 = 3L * (N / 2) * (N / 2) + 1;
-    if (ks.id == KID_UNDO_WINDOW && n >= (1L << 18)) {
-        if (double* tab = (double*)workspace(9, sizeof(double) * N)) {
-            hipLaunchKernelGGL(k_window_factors, dim3(nblk(N)), dim3(256), 0, api_stream(), ks,
-                               N, boxlen, tab);
-            return launch_apply<APPLY_WINDOW>(w, r, N, x0, nx, boxlen, ks, tab);
-        }
-        (void)hipGetLastError();
-    }
-    if ((ks.id == KID_POWER_NO_TRANSFER || ks.id == KID_SQRT_POWER_LAW || ks.id == KID_BBKS) &&
-        n >= (1L << 19) && n >= (ks.id == KID_BBKS ? 2 : 8) * n2) {
-        if (double* tab = (double*)workspace(9, sizeof(double) * n2)) {
-            hipLaunchKernelGGL(k_radial_values, dim3(nblk(n2)), dim3(256), 0, api_stream(), ks,
-                               n2, boxlen, tab);
-            return launch_apply<APPLY_RADIAL>(w, r, N, x0, nx, boxlen, ks, tab);
-        }
-        (void)hipGetLastError();
-    }
-    return launch_apply<APPLY_DIRECT>(w, r, N, x0, nx, boxlen, ks, nullptr);
+    MITOS_TRY((device_apply<TW, TR>(w, r, N, x0, nx, boxlen, ks)));
+    return api_sync();
 }
 
 template <typename T>
@@ -254,15 +261,13 @@ template <typename T>
 bool work_grids(int N, cx<T>** w1, cx<T>** w2, long* hs) {
     const size_t bytes = work_grid_bytes<T>(N), second = bytes <= (32u << 20) ? bytes : 0;
     *hs = work_row<T>(N);
-    *w1 = (cx<T>*)workspace(0, bytes + second);
+    *w1 = (cx<T>*)workspace(SLOT_FFT, bytes + second);
     if (*w1) {
         *w2 = *w1 + second / sizeof(cx<T>);
         return true;
     }
-    (void)hipGetLastError();
     *hs = N / 2 + 1;
-    *w1 = *w2 = (cx<T>*)workspace(0, sizeof(cx<T>) * half_elems(N));
-    if (!*w1) (void)hipGetLastError();
+    *w1 = *w2 = (cx<T>*)workspace(SLOT_FFT, sizeof(cx<T>) * half_elems(N));
     return *w1 != nullptr;
 }
 
@@ -272,6 +277,7 @@ template <typename T, typename OPX>
 int r2c_issue(int N, const T* in, long rs, cx<T>* out, OPX ox) {
     if (!in || !out) return MITOS_ERR_ARG;
     if (!size_supported(N)) return MITOS_ERR_UNSUPPORTED;
+    ScratchLock hold;
     cx<T>*w1, *w2;
     long hs;
     if (!work_grids(N, &w1, &w2, &hs)) w1 = w2 = out;
@@ -283,6 +289,7 @@ template <typename T>
 int c2r_issue(int N, const cx<T>* in, T* out, long rs, double scale) {
     if (!in || !out) return MITOS_ERR_ARG;
     if (!size_supported(N)) return MITOS_ERR_UNSUPPORTED;
+    ScratchLock hold;
     cx<T>*w1, *w2;
     long hs;
     if (!work_grids(N, &w1, &w2, &hs)) return MITOS_ERR_ALLOC;
@@ -557,12 +564,15 @@ extern "C" int solvePoisson_dg(struct distributed_grid* dg) {
 
 extern "C" int solvePoisson(double* phi, double* f, int N, double boxlen) {
     if (!phi || !f) return set_last_error(MITOS_ERR_ARG);
-    cx<double>* fbox = (cx<double>*)workspace(1, sizeof(cx<double>) * half_elems(N));
-    if (!fbox) return set_last_error(MITOS_ERR_ALLOC);
-    const double boxvol = boxlen * boxlen * boxlen;
-    const double s = boxvol / ((long long)N * N * N);
-    MITOS_TRY(set_last_error(
-        (r2c_issue<double>(N, f, N, fbox, OpScalePoisson{N, s, 2 * M_PI / boxlen}))));
-    MITOS_TRY(set_last_error((c2r_issue<double>(N, fbox, phi, N, 1.0 / boxvol))));
+    {
+        ScratchLock hold;
+        cx<double>* fbox = (cx<double>*)workspace(1, sizeof(cx<double>) * half_elems(N));
+        if (!fbox) return set_last_error(MITOS_ERR_ALLOC);
+        const double boxvol = boxlen * boxlen * boxlen;
+        const double s = boxvol / ((long long)N * N * N);
+        MITOS_TRY(set_last_error(
+            (r2c_issue<double>(N, f, N, fbox, OpScalePoisson{N, s, 2 * M_PI / boxlen}))));
+        MITOS_TRY(set_last_error((c2r_issue<double>(N, fbox, phi, N, 1.0 / boxvol))));
+    }
     return set_last_error(api_sync());
 }

@@ -263,30 +263,35 @@ extern "C" int mitos_displace_tsc_dg(const struct distributed_grid* psi_x,
     return set_last_error(api_sync());
 }
 
-extern "C" int mitos_cic_overdensity(int N, double boxlen, long long npart, const float* X,
-                                     const float* Y, const float* Z, double* box) {
-    if (N < 2 || !box || npart <= 0 || !X || !Y || !Z) return set_last_error(MITOS_ERR_ARG);
+static int cic_overdensity_issue(int N, double boxlen, long long npart, const float* X,
+                                 const float* Y, const float* Z, double* box, hipStream_t s) {
     const long ncell = (long)N * N * N;
+    ScratchLock hold;
     unsigned long long* grid =
         (unsigned long long*)workspace(3, sizeof(unsigned long long) * ncell);
-    if (!grid) return set_last_error(MITOS_ERR_ALLOC);
-    hipStream_t s = api_stream();
+    if (!grid) return MITOS_ERR_ALLOC;
     MITOS_HIP_CHECK(hipMemsetAsync(grid, 0, sizeof(unsigned long long) * ncell, s));
     // sorted by tile when that pays and its buffers can be had, else one atomic
     // per corner of every particle: the same integers
     const size_t sort_bytes = cic_sort_bytes(N, npart);
-    void* sort_ws = cic_sort_pays(N, npart, sort_bytes) ? workspace(8, sort_bytes) : nullptr;
-    if (!sort_ws) (void)hipGetLastError();  // no room for the sort: the atomics need none
+    void* sort_ws = cic_sort_pays(N, npart, sort_bytes) ? workspace(SLOT_CIC_SORT, sort_bytes)
+                                                        : nullptr;
     if (sort_ws)
-        MITOS_TRY(set_last_error(
-            cic_sorted<double>(X, Y, Z, npart, N, boxlen, grid, sort_ws, sort_bytes, s)));
+        MITOS_TRY(cic_sorted<double>(X, Y, Z, npart, N, boxlen, grid, sort_ws, sort_bytes, s));
     else
         hipLaunchKernelGGL(k_cic<double>, dim3(nblk(npart)), dim3(256), 0, s, X, Y, Z, npart, N,
                            boxlen, grid);
-    MITOS_TRY(set_last_error(launch_status()));
+    MITOS_TRY(launch_status());
     const double norm = ldexp(1.0, -MITOS_CIC_SHIFT) * ((double)ncell / (double)npart);
     hipLaunchKernelGGL((k_cic_to_delta<double>), dim3(nblk(ncell)), dim3(256), 0, s, grid, box,
                        ncell, (long)N, (long)N, norm);
-    MITOS_TRY(set_last_error(launch_status()));
+    return launch_status();
+}
+
+extern "C" int mitos_cic_overdensity(int N, double boxlen, long long npart, const float* X,
+                                     const float* Y, const float* Z, double* box) {
+    if (N < 2 || !box || npart <= 0 || !X || !Y || !Z) return set_last_error(MITOS_ERR_ARG);
+    MITOS_TRY(set_last_error(
+        cic_overdensity_issue(N, boxlen, npart, X, Y, Z, box, api_stream())));
     return set_last_error(api_sync());
 }

@@ -6,6 +6,7 @@
 
 namespace mitos {
 
+static std::recursive_mutex g_scratch_mu;  // before g_mu
 static std::mutex g_mu;
 static std::map<int, hipStream_t> g_streams;
 static std::map<std::pair<int, int>, std::pair<void*, size_t>> g_ws;
@@ -28,6 +29,11 @@ int api_sync() {
     return MITOS_OK;
 }
 
+ScratchLock::ScratchLock() { g_scratch_mu.lock(); }
+ScratchLock::~ScratchLock() { g_scratch_mu.unlock(); }
+
+static void release_free_blocks_locked();
+
 void* workspace(int slot, size_t bytes) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
@@ -41,7 +47,16 @@ void* workspace(int slot, size_t bytes) {
         g_ws.erase(it);
     }
     void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        hipDeviceSynchronize();
+        release_free_blocks_locked();
+        p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
     g_ws[key] = std::make_pair(p, bytes);
     return p;
 }
@@ -58,25 +73,40 @@ static void release_free_blocks_locked() {
 void* pool_alloc(size_t bytes) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    std::lock_guard<std::mutex> lock(g_mu);
     const auto key = std::make_pair(dev, bytes);
-    auto it = g_free.find(key);
-    if (it != g_free.end()) {
-        void* p = it->second;
-        g_free.erase(it);
-        g_live[p] = key;
-        return p;
-    }
     void* p = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        auto it = g_free.find(key);
+        if (it != g_free.end()) {
+            p = it->second;
+            g_free.erase(it);
+        } else if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            hipDeviceSynchronize();
+            release_free_blocks_locked();
+            if (hipMalloc(&p, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                p = nullptr;
+            }
+        }
+        if (p) {
+            g_live[p] = key;
+            return p;
+        }
+    }
+    ScratchLock hold;
+    std::lock_guard<std::mutex> lock(g_mu);
+    hipDeviceSynchronize();
+    for (int slot : {(int)SLOT_FFT, (int)SLOT_APPLY_TABLE, (int)SLOT_CIC_SORT}) {
+        auto it = g_ws.find(std::make_pair(dev, slot));
+        if (it == g_ws.end()) continue;
+        hipFree(it->second.first);
+        g_ws.erase(it);
+    }
     if (hipMalloc(&p, bytes) != hipSuccess) {
         (void)hipGetLastError();
-        hipDeviceSynchronize();
-        release_free_blocks_locked();
-        p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
+        return nullptr;
     }
     g_live[p] = key;
     return p;
@@ -103,6 +133,7 @@ void pool_trim() {
 }
 
 void release_workspaces() {
+    ScratchLock hold;
     std::lock_guard<std::mutex> lock(g_mu);
     hipDeviceSynchronize();
     for (auto& kv : g_ws) hipFree(kv.second.first);
