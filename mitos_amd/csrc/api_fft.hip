@@ -115,13 +115,17 @@ int apply_transfer(cx<TW>* w, const cx<TR>* r, int N, long x0, long nx, double b
     if (ks < 2 || ts < 2 || !pt->k || !pt->delta || sp->index_src < 0 ||
         sp->index_src >= pt->n_functions || sp->tau_index < 0 || sp->tau_index > ts - 2)
         return MITOS_ERR_ARG;
-    double* d = (double*)workspace(5, sizeof(double) * 3 * ks);
-    if (!d) return MITOS_ERR_ALLOC;
-    const double* rows = pt->delta + (size_t)sp->index_src * ks * ts + (size_t)ks * sp->tau_index;
-    MITOS_HIP_CHECK(copy_sync(d, pt->k, sizeof(double) * ks, hipMemcpyHostToDevice));
-    MITOS_HIP_CHECK(copy_sync(d + ks, rows, sizeof(double) * 2 * ks, hipMemcpyHostToDevice));
-    TransferTab t{d, d + ks, d + 2 * ks, ks, sp->u_tau, invert};
-    MITOS_TRY((issue_apply<APPLY_TRANSFER>(w, r, N, x0, nx, boxlen, KSpec{}, nullptr, t)));
+    {
+        ScratchLock hold;
+        double* d = (double*)workspace(5, sizeof(double) * 3 * ks);
+        if (!d) return MITOS_ERR_ALLOC;
+        const double* rows =
+            pt->delta + (size_t)sp->index_src * ks * ts + (size_t)ks * sp->tau_index;
+        MITOS_HIP_CHECK(copy_sync(d, pt->k, sizeof(double) * ks, hipMemcpyHostToDevice));
+        MITOS_HIP_CHECK(copy_sync(d + ks, rows, sizeof(double) * 2 * ks, hipMemcpyHostToDevice));
+        TransferTab t{d, d + ks, d + 2 * ks, ks, sp->u_tau, invert};
+        MITOS_TRY((issue_apply<APPLY_TRANSFER>(w, r, N, x0, nx, boxlen, KSpec{}, nullptr, t)));
+    }
     return api_sync();
 }
 
