@@ -551,7 +551,7 @@ static int backward(Pipe<T>* P, const mitos_ic_config& cfg, const cx<T>* noise,
         hipLaunchKernelGGL((k_noise_in<T>), dim3(nblk(nh)), dim3(256), 0, s, noise, P->K, hs, N,
                            L, amp);
         MITOS_TRY(launch_status());
-        MITOS_TRY(launch_hermitian<T>(P->K, hs, N, 1, 0, s));
+        MITOS_TRY(launch_hermitian<T>(P->K, hs, N, s));
         T* ph[6] = {reinterpret_cast<T*>(P->b(1)), reinterpret_cast<T*>(P->b(2)),
                     reinterpret_cast<T*>(P->b(3)), reinterpret_cast<T*>(P->b(4)),
                     reinterpret_cast<T*>(P->b(5)), reinterpret_cast<T*>(P->a(2))};

@@ -206,7 +206,7 @@ extern "C" int enforce_hermiticity(struct distributed_grid* dg) {
     if (!dg || !dg->fbox) return set_last_error(MITOS_ERR_ARG);
     hipStream_t s = api_stream();
     MITOS_TRY(set_last_error(launch_hermitian<double>(reinterpret_cast<cx<double>*>(dg->fbox),
-                                                      dg->N / 2 + 1, dg->N, 1, 0, s)));
+                                                      dg->N / 2 + 1, dg->N, s)));
     return set_last_error(api_sync());
 }
 

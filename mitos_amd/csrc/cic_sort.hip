@@ -78,7 +78,7 @@ __global__ void __launch_bounds__(512)
     const int lane = threadIdx.x & 63;
     if (threadIdx.x < 6) box[threadIdx.x] = threadIdx.x < 3 ? 1 << 20 : -1;
     __syncthreads();
-    // tile coordinates, ten bits each (at most 2048 / 8 tiles along an axis)
+    // tile coordinates, ten bits each (at most 4096 / 8 tiles along an axis)
     unsigned tile[K];
     int lo[3] = {1 << 20, 1 << 20, 1 << 20}, hi[3] = {-1, -1, -1};
 #pragma unroll

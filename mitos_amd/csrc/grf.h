@@ -223,8 +223,7 @@ __device__ __forceinline__ cx<T> grf_mode(Xo& gen, const AMP& amp, long n2, doub
 // the stores are 16-mode contiguous runs.
 template <typename T, typename AMP, bool CR>
 __global__ void __launch_bounds__(256)
-    k_grf(cx<T>* out, long hs, int N, double boxlen, long batch_stride, NoiseJumps J,
-          AMP amp) {
+    k_grf(cx<T>* out, long hs, int N, double boxlen, NoiseJumps J, AMP amp) {
     constexpr int ZC = 16;
     __shared__ cx<T> stage[256 * ZC];
     const long nrows = (long)N * N;
@@ -242,7 +241,6 @@ __global__ void __launch_bounds__(256)
     const int WZ = (int)(hz < hs ? hz : hs);
     const int nx = freq_index(x, N), ny = freq_index(y, N);
     const long n2xy = (long)nx * nx + (long)ny * ny;
-    cx<T>* base = out + blockIdx.y * batch_stride;
     for (int z0 = 0; z0 < H; z0 += ZC) {
         if (ok) {
             for (int dz = 0; dz < ZC; dz++) {
@@ -268,7 +266,7 @@ __global__ void __launch_bounds__(256)
             const int idx = i * 256 + threadIdx.x;
             const int r = idx / ZC, dz = idx % ZC;
             const long l = line0 + r;
-            if (l < nrows && z0 + dz < WZ) st(base + l * hs + z0 + dz, stage[r * ZC + dz]);
+            if (l < nrows && z0 + dz < WZ) st(out + l * hs + z0 + dz, stage[r * ZC + dz]);
         }
         __syncthreads();
     }
@@ -356,7 +354,7 @@ __global__ void __launch_bounds__(256)
 // src/grf.c:78-175 on one rank.  In place: every lower-half point reads its
 // mirror, which lies in the untouched upper half or is the point itself.
 template <typename T>
-__global__ void k_hermitian(cx<T>* f, long hs, int N, long batch_stride) {
+__global__ void k_hermitian(cx<T>* f, long hs, int N) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long per = (long)(N / 2 + 1) * N;
     if (i >= 2 * per) return;
@@ -367,13 +365,12 @@ __global__ void k_hermitian(cx<T>* f, long hs, int N, long batch_stride) {
     const int invx = (x > 0) ? N - x : 0;
     const int invy = (y > 0) ? N - y : 0;
     const int invz = (z > 0) ? N - z : 0;
-    cx<T>* g = f + blockIdx.y * batch_stride;
     const long id = ((long)x * N + y) * hs + z;
     if (invx == x && invy == y && invz == z) {
-        g[id].im = 0;
+        f[id].im = 0;
     } else {
         const long mid = ((long)invx * N + invy) * hs + z;
-        g[id] = conjg(g[mid]);
+        f[id] = conjg(f[mid]);
     }
 }
 
@@ -416,15 +413,15 @@ int launch_grf(cx<T>* out, long hs, int N, double boxlen, const NoiseJumps& J, A
         }
     }
     hipLaunchKernelGGL((k_grf<T, AMP, CR>), dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s,
-                       out, hs, N, boxlen, 0L, J, amp);
+                       out, hs, N, boxlen, J, amp);
     return hipGetLastError() == hipSuccess ? MITOS_OK : MITOS_ERR_DEVICE;
 }
 
 template <typename T>
-int launch_hermitian(cx<T>* f, long hs, int N, int nb, long bstride, hipStream_t s) {
+int launch_hermitian(cx<T>* f, long hs, int N, hipStream_t s) {
     const long n = 2L * (N / 2 + 1) * N;
-    dim3 grid((unsigned)((n + 255) / 256), nb);
-    hipLaunchKernelGGL((k_hermitian<T>), grid, dim3(256), 0, s, f, hs, N, bstride);
+    hipLaunchKernelGGL((k_hermitian<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, f, hs,
+                       N);
     return hipGetLastError() == hipSuccess ? MITOS_OK : MITOS_ERR_DEVICE;
 }
 

@@ -53,9 +53,11 @@ struct MultiK<T, L, AXIS, DIR, NIN, CODES, Radices<Rs...>> {
 // Lines of k_hess_z: in FP64 four values a thread for powers of two, so the four
 // arrays of a thread's row leave room for its addresses and twiddles, and a row of
 // 256 is one wave, whose barriers wait on nobody (rows of fewer threads share a
-// wave).  Against eight a thread: 512^3 3.05 -> 2.14 ms, the drop-in 2LPT at 256^3
-// 1.80 -> 1.70 ms.  Bound by latency at two waves a SIMD: four waves (addresses and
-// twiddles formed anew per row) took 2.33 ms at 512^3 and 1.80 ms.
+// wave).  Against eight a thread, by the realization's own stage times: 128^3 48 -> 37
+// us, 256^3 341 -> 247 us, 512^3 2.61 -> 1.65 ms, 1024^3 16.2 -> 15.0 ms (lines of 64 to
+// 512); the drop-in 2LPT at 256^3 1.80 -> 1.66 ms.  Bound by latency at two waves a
+// SIMD: four waves (addresses and twiddles formed anew per row) were slower (512^3 2.33
+// against 2.14 ms under the profiler).
 template <typename T, int L>
 struct HessCfg : LineCfgS<L> {};
 template <>

@@ -1358,10 +1358,9 @@ __host__ __device__ __forceinline__ void cic_cell_t(T x, T icell, int N, int& i,
     i = (unsigned)i < (unsigned)N ? i : wrapi(i, N);
 }
 
-// Lattice site of thread t's particle j in the order of the adjoint's particle
-// kernels: work-groups of 256 threads over 8 x 8 x 16 tiles (x, y, z), four
-// particles a thread, so the taps of a work-group share lines in L1.  False
-// past the grid's edge (N = 8, 24).
+// First site of work-group b of the adjoint's particle kernels: tiles of 8 x 8 x 16
+// sites (x, y, z), so the taps of a work-group share lines in L1.  N is a multiple of 8;
+// the last tile of a z row may reach past the grid (N = 8, 24).
 constexpr int kAdjTX = 8, kAdjTY = 8, kAdjTZ = 16;
 inline unsigned adj_tiles(int N) {
     return (unsigned)((N / kAdjTX) * (N / kAdjTY) * ((N + kAdjTZ - 1) / kAdjTZ));

@@ -190,7 +190,7 @@ int Pipe<T>::enqueue(const mitos_ic_config& cfg, hipStream_t s, bool timing,
         return launch_grf<T, AmpTable, sizeof(T) == 8>(K, hs, N, L, J, AmpTable{amp}, s);
     }));
     MITOS_TRY(timed(s, "hermitian_planes", 0.0,
-                    [&] { return launch_hermitian<T>(K, hs, N, 1, 0, s); }));
+                    [&] { return launch_hermitian<T>(K, hs, N, s); }));
     mark(1);
     return with_size(N, [&]<int NN>() -> int {
         cx<T>* D = a(0);
